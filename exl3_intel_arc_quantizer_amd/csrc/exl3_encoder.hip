@@ -913,42 +913,56 @@ struct TbArgs {
 //
 // Leaf n = k_0 .. k_D (k_D least significant) lives in lane n >> RLOG,
 // register n & (R - 1), R = 2^RLOG leaves per lane, so the lowest digits are
-// reduced inside a lane and a lane's leaves are one aligned vector load.
-// Once a level has reduced every register bit, the registers of a lane hold
-// copies of one value and the remaining digits reduce across lanes with
-// xor_min (DPP / permlane swaps). Trees with fewer than 64 leaves are
-// replicated over the wave.
+// reduced inside a lane and a lane's leaves are one aligned vector load. The
+// remaining digits reduce across lanes, lowest lane bit first. Trees with
+// fewer than 64 leaves are replicated over the wave.
+//
+// The walk is one serial chain per tile (load a tree, evaluate it, find the
+// next edge), bound by that chain's latency: at 64 tiles, one wave on its
+// own, it took 0.44 us per stored row at K = 4. So everything that does not
+// depend on the lane is uniform (edge, row address and step live in scalar
+// registers, the branches are scalar), what does not depend on the edge is
+// computed once per walk (each lane's part of the leaf address and of every
+// level's codebook hash: both are linear over the disjoint bits of lane and
+// edge), leaves are decoded and evaluated in packed pairs, and a level's
+// lane reduction takes one DPP minimum per lane bit.
 
-// min(v, v of lane ^ mask) for mask = 1 .. 32 without the LDS crossbar:
-// DPP quad_perm (1, 2), quad reversal then row_half_mirror (4: i ^ 3 ^ 7),
-// row_ror:8 (8), and gfx950's v_permlane16_swap / v_permlane32_swap (16,
-// 32: the swapped pair holds each lane's value and its partner's). mask
-// must fold to a constant; every lane of the wave must be active.
-__device__ __forceinline__ uint32_t dpp_mov(uint32_t v, int ctrl) {
-  switch (ctrl) {
-    case 0xB1: return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, false);
-    case 0x4E: return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, false);
-    case 0x1B: return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x1B, 0xF, 0xF, false);
-    case 0x141: return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, false);
-    default: return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xF, 0xF, false);
+// min(v, v of the lane whose index differs in bit B), one DPP instruction
+// each, for lanes whose lower index bits hold copies of one value: quad_perm
+// (bits 0, 1), row_half_mirror (bit 2: i ^ 7, the other quad) and row_ror:8
+// (bit 3). Bits 4 and 5 reduce towards the highest lane: row_bcast:15 takes
+// lane 15 of each even row into the odd row after it (afterwards rows 1 and
+// 3 are valid), row_bcast:31 lane 31 into rows 2 and 3 (row 3 is valid).
+template <int B>
+__device__ __forceinline__ uint32_t lane_bit_min(uint32_t v) {
+  constexpr int kCtrl[6] = {0xB1, 0x4E, 0x141, 0x128, 0x142, 0x143};
+  constexpr int kRows[6] = {0xF, 0xF, 0xF, 0xF, 0xA, 0xC};
+  // Lanes outside the row mask keep their own value (old = the identity).
+  return umin(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, kCtrl[B], kRows[B], 0xF, false));
+}
+
+template <int B0, int B1>
+__device__ __forceinline__ uint32_t lane_bits_min(uint32_t v) {
+  if constexpr (B0 < B1) {
+    return lane_bits_min<B0 + 1, B1>(lane_bit_min<B0>(v));
+  } else {
+    return v;
   }
 }
 
-__device__ __forceinline__ uint32_t xor_min(uint32_t v, int mask) {
-  switch (mask) {
-    case 1: return umin(v, dpp_mov(v, 0xB1));
-    case 2: return umin(v, dpp_mov(v, 0x4E));
-    case 4: return umin(v, dpp_mov(dpp_mov(v, 0x1B), 0x141));
-    case 8: return umin(v, dpp_mov(v, 0x128));
-    case 16: {
-      const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-      return umin(r[0], r[1]);
-    }
-    default: {
-      const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-      return umin(r[0], r[1]);
-    }
+// fp16 values of two hashed states.
+__device__ __forceinline__ f16x2 decode_hash_pair(int cb, uint32_t x0, uint32_t x1) {
+  if (cb == 2) {
+    // The two byte sums accumulate onto the halves of 0x64006400 (see
+    // decode_hash; a sum is at most 1020, so the low half does not carry).
+    const uint32_t h =
+        __builtin_amdgcn_sad_hi_u8(x1, 0u, __builtin_amdgcn_sad_u8(x0, 0u, 0x64006400u));
+    const f16 a = f16_bits(0x1EEEu), b = f16_bits(0xC931u);
+    const f16x2 a2 = {a, a}, b2 = {b, b};
+    return __builtin_elementwise_fma(__builtin_bit_cast(f16x2, h), a2, b2);
   }
+  const f16x2 v = {decode_hash(cb, x0), decode_hash(cb, x1)};
+  return v;
 }
 
 template <int N>
@@ -961,495 +975,408 @@ __device__ __forceinline__ uint32_t row_pos(uint32_t x) {
   return exl3::cost_row_pos(K, x);
 }
 
-// The states a traceback tree decodes, split into the part that depends on
-// the lane (and the walk's edge) and the part that depends on the register
-// index r. Leaf n = (lane << RLOG | r) & (2^(K(D+1)) - 1); every bit of the
-// state at level m is a copy of one bit of n or of the edge, so the state is
-// the disjoint OR (= sum) of its value with r = 0 and its value with lane = 0
-// and edge = 0. hash_state is affine, so the hash of the leaf's state is the
-// lane's hash (one multiply per level) plus a compile-time offset per r.
-template <int K, int D, int RLOG>
-struct TreeFields {
-  static constexpr int NB = 1 << K, KR = 16 - K, KS = 16 - 2 * K;
-  static constexpr int NLOG = K * (D + 1);
-  static constexpr uint32_t NMASK = (1u << NLOG) - 1u;
-  uint32_t nl, h0;
-
-  __device__ __forceinline__ TreeFields(int lane, uint32_t edge_hi)
-      : nl(((uint32_t)lane << RLOG) & NMASK), h0(edge_hi) {}
-
-  // x_m of leaf n (the predecessor edge at level m) with edge part hh.
-  __host__ __device__ static constexpr uint32_t x_at(uint32_t n, uint32_t hh, int m) {
-    uint32_t x = ((n >> (K * D)) << KS) | hh;
-    for (int j = 1; j <= m; ++j) x = (((n >> (K * (D - j))) & (NB - 1)) << KS) | (x >> K);
-    return x;
-  }
-  // State decoded at level m (digit k_{m+1} over x_m).
-  __host__ __device__ static constexpr uint32_t level_state(uint32_t n, uint32_t hh, int m) {
-    const int lo = K * (D - 1 - m);
-    return (((n >> lo) & (NB - 1)) << KR) | x_at(n, hh, m);
-  }
-  __device__ __forceinline__ uint32_t level_hash(int cb, int m) const {
-    return hash_state(cb, level_state(nl, h0, m));
-  }
-  __host__ __device__ static constexpr uint32_t level_offset(int cb, int m, int r) {
-    return level_state((uint32_t)r & NMASK, 0u, m) * hash_mult(cb);
-  }
-  // State decoded at the top (digit k_0 over the walk's edge).
-  __device__ __forceinline__ uint32_t top_hash(int cb, uint32_t edge) const {
-    return hash_state(cb, ((nl >> (K * D)) << KR) | edge);
-  }
-  __host__ __device__ static constexpr uint32_t top_offset(int cb, int r) {
-    return ((((uint32_t)r & NMASK) >> (K * D)) << KR) * hash_mult(cb);
-  }
-};
-
-template <int K, int CB, int D, bool INIT>
-__device__ __forceinline__ uint32_t tb_branch(const uint16_t* __restrict__ leaf, uint32_t edge,
-                                              const uint16_t* __restrict__ wbits, int ri, int L,
-                                              int lane, int pre) {
-  constexpr int NB = 1 << K, KS = 16 - 2 * K;
-  constexpr int NLOG = K * (D + 1);
-  constexpr int RLOG = NLOG > 6 ? NLOG - 6 : 0;
-  constexpr int R = 1 << RLOG;
-  constexpr uint32_t NMASK = (1u << NLOG) - 1u;
-  constexpr int CH = R < NB ? R : NB;  // leaves per contiguous load
-  const uint32_t h0 = edge >> K;
-
-  uint32_t nid[R];
-  uint32_t xs[R][D + 1];
-  uint32_t v[R];
-  TreeFields<K, D, RLOG> tf(lane, h0);
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const uint32_t n = (((uint32_t)lane << RLOG) | (uint32_t)r) & NMASK;
-    nid[r] = n;
-    uint32_t x = ((n >> (K * D)) << KS) | h0;
-    xs[r][0] = x;
-#pragma unroll
-    for (int m = 1; m <= D; ++m) {
-      x = (((n >> (K * (D - m))) & (NB - 1)) << KS) | (x >> K);
-      xs[r][m] = x;
-    }
-  }
-  if constexpr (INIT) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) v[r] = (pre < 0 || (int)xs[r][0] == pre) ? 0u : 0x7C00u;
-  } else {
-#pragma unroll
-    for (int c = 0; c < R / CH; ++c) {
-      const typename U16Vec<CH>::type q =
-          *reinterpret_cast<const typename U16Vec<CH>::type*>(leaf + nid[c * CH]);
-#pragma unroll
-      for (int u = 0; u < CH; ++u) v[c * CH + u] = q[u];
-    }
-  }
-
-  // Levels D-1 .. 0: reduce digit k_{m+1}, bits [lo, lo + K) of n.
-#pragma unroll
-  for (int m = D - 1; m >= 0; --m) {
-    const int lo = K * (D - 1 - m), hi = lo + K;
-    int rm = ri - 1 - m;
-    if (rm < 0) rm += L;
-    const f16 wm = f16_bits(wbits[rm]);
-    const int nr = lo < RLOG ? R : 1;  // registers still distinct
-    const uint32_t hl = tf.level_hash(CB, m);
-#pragma unroll
-    for (int r = 0; r < nr; ++r) {
-      const f16 dh = decode_hash(CB, hl + TreeFields<K, D, RLOG>::level_offset(CB, m, r)) - wm;
-      v[r] = bits_f16(__builtin_fmaf16(dh, dh, f16_bits(v[r])));
-    }
-#pragma unroll
-    for (int b = lo; b < (hi < RLOG ? hi : RLOG); ++b)
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-        if (!(r & (1 << b))) {
-          const uint32_t t = umin(v[r], v[r | (1 << b)]);
-          v[r] = t;
-          v[r | (1 << b)] = t;
-        }
-    if (hi > RLOG) {
-#pragma unroll
-      for (int b = (lo > RLOG ? lo : RLOG); b < (hi < NLOG ? hi : NLOG); ++b)
-        v[0] = xor_min(v[0], 1 << (b - RLOG));
-#pragma unroll
-      for (int r = 1; r < R; ++r) v[r] = v[0];
-    }
-  }
-
-  // Step i: key minimum over k_0, bits [K D, NLOG) of n.
-  const f16 w = f16_bits(wbits[ri]);
-  const int nr = (K * D) < RLOG ? R : 1;
-  const uint32_t ht = tf.top_hash(CB, edge);
-  uint32_t key = 0xFFFFFFFFu;
-#pragma unroll
-  for (int r = 0; r < nr; ++r) {
-    const uint32_t k0 = nid[r] >> (K * D);
-    const f16 dh = decode_hash(CB, ht + TreeFields<K, D, RLOG>::top_offset(CB, r)) - w;
-    const f16 err = __builtin_fmaf16(dh, dh, f16_bits(v[r]));
-    key = umin(key, ((uint32_t)bits_f16(err) << 16) | k0);
-  }
-#pragma unroll
-  for (int b = (K * D > RLOG ? K * D : RLOG); b < NLOG; ++b)
-    key = xor_min(key, 1 << (b - RLOG));
-  return key & 0xFFFFu;
-}
+constexpr int cmin(int a, int b) { return a < b ? a : b; }
+constexpr int cmax(int a, int b) { return a > b ? a : b; }
 
 // The decisions of every step that reads one stored row, from one
 // evaluation of the row's depth-D tree. Step i's choice is the key minimum
 // at the top; the level-m reduction computes exactly what step i-1-m
 // chooses between (the FMA over its 2^K predecessors, whose costs are the
-// level below), so if each level reduces keys (cost_bits << 16) | digit
-// instead of bare costs, the choice of step i-1-m for the prefix chosen
-// above is the digit of the level-m key held by that prefix's lane and
-// register (lowest digit on equal costs, as the forward pass). Returns the
-// branches packed: bits [K j, K j + K) hold the branch of step i - j,
-// j = 0..D (K * row_stride(K) <= 10 bits).
+// level below). A level reduces keys (cost_bits << 16) | digits, where
+// digits is the candidate's own digit k_{m+1} above the digits its own
+// minimum chose below it: equal costs resolve to the lowest k_{m+1}, as in
+// the forward pass, and the winning key at the top carries the whole path
+// (K (D + 1) <= 10 bits).
 //
-// The leaves are read straight from the stored row (HBM, or an LDS copy of
-// it): leaf n sits at row_pos(x_D(n)), and a lane's CH leaves that differ
-// only in the last digit are one aligned vector of siblings.
-template <int K, int CB, int D>
-__device__ __forceinline__ uint32_t tb_tree(const uint16_t* __restrict__ row, uint32_t edge,
-                                            const uint16_t* __restrict__ wbits, int ri, int L,
-                                            int lane) {
-  constexpr int NB = 1 << K, KS = 16 - 2 * K;
-  constexpr int NLOG = K * (D + 1);
-  constexpr int RLOG = NLOG > 6 ? NLOG - 6 : 0;
-  constexpr int R = 1 << RLOG;
-  constexpr uint32_t NMASK = (1u << NLOG) - 1u;
-  // A lane's R leaves are one aligned run in K = 2's tree-major rows, and
-  // its 2^K siblings elsewhere.
-  constexpr int CH = (K == 2 || K == 3 || R < NB) ? R : NB;
-  const uint32_t h0 = edge >> K;
-
-  uint32_t nid[R];
-  uint32_t xs[R][D + 1];
-  uint32_t v[R];
-  TreeFields<K, D, RLOG> tf(lane, h0);
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const uint32_t n = (((uint32_t)lane << RLOG) | (uint32_t)r) & NMASK;
-    nid[r] = n;
-    uint32_t x = ((n >> (K * D)) << KS) | h0;
-    xs[r][0] = x;
-#pragma unroll
-    for (int m = 1; m <= D; ++m) {
-      x = (((n >> (K * (D - m))) & (NB - 1)) << KS) | (x >> K);
-      xs[r][m] = x;
-    }
-  }
-#pragma unroll
-  for (int c = 0; c < R / CH; ++c) {
-    const typename U16Vec<CH>::type q = *reinterpret_cast<const typename U16Vec<CH>::type*>(
-        row + row_pos<K>(xs[c * CH][D]));
-#pragma unroll
-    for (int u = 0; u < CH; ++u) v[c * CH + u] = q[u];
-  }
-  // A lane's leaves are at most 8 bytes (R <= 4) at every K but 2, whose
-  // 16 (32 bytes, two loads) are one aligned run.
+// Leaf n sits at row_pos(x_D(n)) of the stored row, and a lane's CH leaves
+// that differ only in its lowest bits are one aligned vector. INIT (D = 0):
+// step 0, whose predecessor costs are the start constraint, not a row.
+template <int K, int CB, int D, bool INIT = false>
+struct Tree {
+  static constexpr int NB = 1 << K, KR = 16 - K, KS = 16 - 2 * K;
+  static constexpr int NLOG = K * (D + 1);
+  static constexpr int RLOG = cmax(NLOG - 6, 0), R = 1 << RLOG;
+  static constexpr uint32_t NMASK = (1u << NLOG) - 1u;
+  // A lane's R leaves are one aligned run in the tree-major rows (K = 2, 3),
+  // and its 2^K siblings elsewhere.
+  static constexpr int CH = (K == 2 || K == 3 || R < NB) ? R : NB;
   static_assert(R <= 4 || ((K == 2 || K == 3) && R <= 16), "a lane's leaves are one run");
+  static_assert(NLOG <= 16, "a path's digits fit below the cost bits");
 
-  uint32_t lvl[D > 0 ? D : 1][R];
+  // x_m of leaf n (the predecessor edge at level m) for edge 0.
+  __host__ __device__ static constexpr uint32_t x_at(uint32_t n, int m) {
+    uint32_t x = (n >> (K * D)) << KS;
+    for (int j = 1; j <= m; ++j) x = (((n >> (K * (D - j))) & (NB - 1)) << KS) | (x >> K);
+    return x;
+  }
+  // Leaf n's part of the state decoded at level m (digit k_{m+1} over x_m;
+  // m = -1: digit k_0 over the walk's edge). The edge's part is the disjoint
+  // edge >> K (m + 1).
+  __host__ __device__ static constexpr uint32_t level_state(uint32_t n, int m) {
+    return (((n >> (K * (D - 1 - m))) & (NB - 1)) << KR) | (m < 0 ? 0u : x_at(n, m));
+  }
+
+  uint32_t nl;        // leaf index of the lane's register 0
+  uint32_t leaf_off;  // its position in a row, edge 0
+  uint32_t lane_hash[D + 1];  // its hash at level m, edge 0, in lane_hash[m + 1]
+  __device__ __forceinline__ explicit Tree(int lane) {
+    nl = ((uint32_t)lane << RLOG) & NMASK;
+    leaf_off = INIT ? 0u : row_pos<K>(x_at(nl, D));
 #pragma unroll
-  for (int m = D - 1; m >= 0; --m) {
-    const int lo = K * (D - 1 - m), hi = lo + K;
-    int rm = ri - 1 - m;
-    if (rm < 0) rm += L;
-    const f16 wm = f16_bits(wbits[rm]);
-    const int nr = lo < RLOG ? R : 1;  // registers still distinct
-    const uint32_t hl = tf.level_hash(CB, m);
+    for (int m = -1; m < D; ++m) lane_hash[m + 1] = hash_state(CB, level_state(nl, m));
+  }
+
+  // Level M (M = -1: the top) over the distinct entries [0 .. IN) of the
+  // level below: err = fma(dh, dh, cost), costs the entries' fp16 costs and
+  // below their keys (none at the leaves), reduced over the level's digit
+  // into key[0 .. OUT).
+  template <int M>
+  __device__ __forceinline__ void level(const f16* cost, const uint32_t* below, uint32_t edge,
+                                        f16 w, uint32_t* key) const {
+    constexpr int LO = K * (D - 1 - M), HI = LO + K;
+    constexpr int IN = R >> cmin(LO, RLOG), OUT = R >> cmin(HI, RLOG), G = IN / OUT;
+    const uint32_t h = lane_hash[M + 1] + (edge >> (K * (M + 1))) * hash_mult(CB);
+    const uint32_t lane_digit = nl & ((NB - 1u) << LO);
+    uint32_t full[IN];
 #pragma unroll
-    for (int r = 0; r < nr; ++r) {
-      const uint32_t k = (nid[r] >> lo) & (NB - 1);
-      const f16 dh = decode_hash(CB, hl + TreeFields<K, D, RLOG>::level_offset(CB, m, r)) - wm;
-      v[r] = ((uint32_t)bits_f16(__builtin_fmaf16(dh, dh, f16_bits(v[r]))) << 16) | k;
+    for (int x = 0; x < IN; ++x) {
+      // The entry's digits, its own at bit LO: register index x << LO.
+      full[x] = lane_digit | ((x & (NB - 1u)) << LO);
+      if (LO > 0) full[x] |= below[x] & 0xFFFFu;
     }
-    if (nr == 1) {
+    if constexpr (IN == 1) {
+      const f16 dh = decode_hash(CB, h) - w;
+      const f16 e = __builtin_fmaf16(dh, dh, cost[0]);
+      full[0] |= (uint32_t)bits_f16(e) << 16;
+    } else {
+      const f16x2 w2 = {w, w};
 #pragma unroll
-      for (int r = 1; r < R; ++r) v[r] = v[0];
+      for (int x = 0; x < IN; x += 2) {
+        const f16x2 c2 = {cost[x], cost[x + 1]};
+        const f16x2 dh =
+            decode_hash_pair(CB, h + level_state((uint32_t)x << LO, M) * hash_mult(CB),
+                             h + level_state((uint32_t)(x + 1) << LO, M) * hash_mult(CB)) - w2;
+        const uint32_t e = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(dh, dh, c2));
+        full[x] |= e << 16;
+        full[x + 1] |= e & 0xFFFF0000u;
+      }
     }
 #pragma unroll
-    for (int b = lo; b < (hi < RLOG ? hi : RLOG); ++b)
+    for (int o = 0; o < OUT; ++o) {
+      uint32_t k = full[o * G];
 #pragma unroll
-      for (int r = 0; r < R; ++r)
-        if (!(r & (1 << b))) {
-          const uint32_t t = umin(v[r], v[r | (1 << b)]);
-          v[r] = t;
-          v[r | (1 << b)] = t;
-        }
-    if (hi > RLOG) {
-#pragma unroll
-      for (int b = (lo > RLOG ? lo : RLOG); b < (hi < NLOG ? hi : NLOG); ++b)
-        v[0] = xor_min(v[0], 1 << (b - RLOG));
-#pragma unroll
-      for (int r = 1; r < R; ++r) v[r] = v[0];
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      lvl[m][r] = v[r];
-      v[r] >>= 16;
+      for (int g = 1; g < G; ++g) k = umin(k, full[o * G + g]);
+      key[o] = lane_bits_min<cmax(LO - RLOG, 0), cmax(HI - RLOG, 0)>(k);
     }
   }
 
-  // Step i: key minimum over k_0, bits [K D, NLOG) of n.
-  const f16 w = f16_bits(wbits[ri]);
-  const int nr = (K * D) < RLOG ? R : 1;
-  const uint32_t ht = tf.top_hash(CB, edge);
-  uint32_t key = 0xFFFFFFFFu;
+  // Levels D-1 .. M, bottom up, then the top (M = -1).
+  template <int M>
+  __device__ __forceinline__ void levels(f16* cost, uint32_t* key, uint32_t edge,
+                                         const f16* w) const {
+    if constexpr (M < D) {
+      levels<M + 1>(cost, key, edge, w);
+      uint32_t out[R];
+      level<M>(cost, key, edge, w[M + 1], out);
+      constexpr int OUT = R >> cmin(K * (D - M), RLOG);
 #pragma unroll
-  for (int r = 0; r < nr; ++r) {
-    const uint32_t k0 = nid[r] >> (K * D);
-    const f16 dh = decode_hash(CB, ht + TreeFields<K, D, RLOG>::top_offset(CB, r)) - w;
-    const f16 err = __builtin_fmaf16(dh, dh, f16_bits(v[r]));
-    key = umin(key, ((uint32_t)bits_f16(err) << 16) | k0);
-  }
-#pragma unroll
-  for (int b = (K * D > RLOG ? K * D : RLOG); b < NLOG; ++b)
-    key = xor_min(key, 1 << (b - RLOG));
-  uint32_t prefix = (uint32_t)__builtin_amdgcn_readfirstlane((int)key) & 0xFFFFu;
-  uint32_t ks = prefix;
-#pragma unroll
-  for (int m = 0; m < D; ++m) {
-    const uint32_t nsel = prefix << (K * (D - m));  // the prefix's first leaf
-    const int reg = (int)(nsel & (uint32_t)(R - 1));
-    uint32_t sel = lvl[m][0];
-#pragma unroll
-    for (int r = 1; r < R; ++r)
-      if (r == reg) sel = lvl[m][r];
-    const uint32_t kk =
-        (uint32_t)__builtin_amdgcn_readlane((int)sel, (int)(nsel >> RLOG)) & 0xFFFFu;
-    ks |= kk << (K * (m + 1));
-    prefix = (prefix << K) | kk;
-  }
-  return ks;
-}
-
-template <int K, int CB, int D>
-__device__ __forceinline__ uint32_t tb_tree_dispatch(int d, const uint16_t* row, uint32_t edge,
-                                                     const uint16_t* __restrict__ wbits, int ri,
-                                                     int L, int lane) {
-  static_assert(K * exl3::row_stride(K) <= 32, "a row's branches fit in one word");
-  if constexpr (D + 1 < exl3::row_stride(K)) {
-    if (d != D) return tb_tree_dispatch<K, CB, D + 1>(d, row, edge, wbits, ri, L, lane);
-  }
-  return tb_tree<K, CB, D>(row, edge, wbits, ri, L, lane);
-}
-
-// One stored row serves steps i .. r0 + 1: its tree is loaded once, at the
-// first of them, and evaluated once (tb_tree), which yields all of their
-// branches. One dependent HBM load and one tree evaluation per stride of
-// steps.
-template <int K, int CB>
-__global__ void __launch_bounds__(64) traceback_rows_kernel(TbArgs a) {
-  constexpr int KR = 16 - K;
-  constexpr int STRIDE = exl3::row_stride(K);
-  __shared__ uint16_t s_wbits[256];  // the tile's fp16 inputs, ring order
-  __shared__ uint16_t s_oidx[256];   // the walk's states, ring order (write pass)
-  const int t = blockIdx.x;
-  const int lane = threadIdx.x;
-  const int L = a.L;
-  const uint8_t* blk = a.scratch + (int64_t)t * a.tile_stride;
-  const uint8_t* hdr = blk + a.hdr_offset;
-  const int row_bytes = a.lay.row_bytes;
-  const int pre = reinterpret_cast<const int32_t*>(hdr)[exl3::HDR_PRE_STATE];
-  const uint16_t* wsrc = reinterpret_cast<const uint16_t*>(hdr + exl3::HDR_W_BYTES);
-  for (int r = lane; r < L; r += 64) s_wbits[r] = wsrc[r];
-  __syncthreads();
-  const uint16_t* wbits = s_wbits;
-  uint32_t edge = (uint32_t)a.start[(int64_t)t * a.start_stride] & ((65536u >> K) - 1u);
-  const int i_stop = a.write ? 0 : (L - a.roll) % L;  // the last step walked
-
-  int i = L - 1;
-  while (i >= 1 && i >= i_stop) {
-    // Steps i .. r0 + 1 read stored row r0: one tree load, one evaluation.
-    const int d = (i - 1) % STRIDE;
-    const int r0 = i - 1 - d;
-    const uint16_t* row =
-        reinterpret_cast<const uint16_t*>(blk + (int64_t)(r0 / STRIDE) * row_bytes);
-    int ri = i + a.roll;
-    if (ri >= L) ri -= L;
-    const uint32_t ks = tb_tree_dispatch<K, CB, 0>(d, row, edge, wbits, ri, L, lane);
-#pragma unroll
-    for (int j = 0; j < STRIDE; ++j) {
-      if (j <= d && i >= i_stop) {
-        int rj = i + a.roll;
-        if (rj >= L) rj -= L;
-        const uint32_t sigma = (((ks >> (K * j)) & ((1u << K) - 1u)) << KR) | edge;
-        if (a.write && lane == 0) s_oidx[rj] = (uint16_t)sigma;
-        edge = sigma >> K;
-        --i;
+      for (int o = 0; o < OUT; ++o) {
+        key[o] = out[o];
+        cost[o] = f16_bits(out[o] >> 16);
       }
     }
   }
-  if (i == 0 && i_stop == 0) {  // step 0: predecessors from the start constraint
-    int ri = a.roll;
-    if (ri >= L) ri -= L;
-    const uint32_t k = tb_branch<K, CB, 0, true>(nullptr, edge, wbits, ri, L, lane, pre);
-    const uint32_t sigma = (k << KR) | edge;
-    if (a.write && lane == 0) s_oidx[ri] = (uint16_t)sigma;
-    edge = sigma >> K;
-  }
-  if (a.write) {
-    // The states and their codebook values leave after the walk, coalesced
-    // over the wave, so the serial walk carries no decode or global store.
-    __syncthreads();
-    for (int r = lane; r < L; r += 64) {
-      const uint32_t sigma = s_oidx[r];
-      a.out_idx[(int64_t)t * L + r] = (int16_t)(uint16_t)sigma;
-      a.out_w[(int64_t)t * L + r] = (float)decode_state(CB, sigma);
+
+  // Digits k_0 .. k_D, k_0 most significant, with k_0 moved to the bottom.
+  __device__ __forceinline__ static uint32_t reverse_digits(uint32_t n) {
+    if constexpr (D == 0) {
+      return n;
+    } else if constexpr (K == 1) {
+      return __builtin_bitreverse32(n) >> (32 - NLOG);
+    } else if constexpr (K == 2) {
+      const uint32_t b = __builtin_bitreverse32(n) >> (32 - NLOG);
+      return ((b & 0x55555555u) << 1) | ((b >> 1) & 0x55555555u);
+    } else {
+      uint32_t ks = 0;
+#pragma unroll
+      for (int j = 0; j <= D; ++j) ks |= ((n >> (K * (D - j))) & (NB - 1)) << (K * j);
+      return ks;
     }
-  } else if (lane == 0) {
-    a.end_out[(int64_t)t * a.end_stride] = (int32_t)edge;
   }
-}
 
-// Streamed cost-row traceback for small batches. The traceback above is
-// bound by one dependent HBM load per stored row and tile; with few tiles
-// in flight that latency is the whole kernel. Here one workgroup per tile
-// streams every stored row it will visit into a two-slot LDS ring ahead of
-// the walk (the rows are known in advance, only the tree inside a row
-// depends on the path): wave 0 walks exactly as traceback_rows_kernel,
-// reading its trees from the ring; NG loader groups of W waves take rows in
-// turn (row j belongs to group j % NG), so a row's load has NG rows of walk
-// time to arrive while every group keeps one row in statically indexed
-// registers. One workgroup barrier per stored row, LDS-only fences so loads
-// stay in flight across it. Reads every row whole (E x 2 bytes instead of
-// one tree), so it pays off only while HBM bandwidth is idle.
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-template <int K>
-struct StreamShape {
-  static constexpr int W = (K == 1 || K == 2) ? 4 : (K <= 4 ? 2 : 1);  // waves per group
-  static constexpr int NG = (K == 1) ? 1 : (K == 2 ? 2 : (K <= 5 ? 4 : 8));
-  static_assert(K >= 1 && K <= 8, "cost-row bitrates");
-  static constexpr int THREADS = 64 * (1 + W * NG);
+  // The branches of steps i .. i - D for the walk's edge (uniform) at step
+  // i, packed: bits [K j, K j + K) hold the branch of step i - j. w[j] is
+  // the input of step i - j.
+  __device__ __forceinline__ uint32_t branches(const uint16_t* row, uint32_t edge, const f16* w,
+                                               int pre) const {
+    f16 cost[R];
+    if constexpr (INIT) {
+      static_assert(D == 0, "step 0 reads no row");
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int x = (int)(((nl | r) << KS) | (edge >> K));
+        cost[r] = f16_bits((pre < 0 || x == pre) ? 0u : 0x7C00u);
+      }
+    } else {
+      const uint16_t* base = row + row_pos<K>(edge >> NLOG);
+#pragma unroll
+      for (int c = 0; c < R; c += CH) {
+        const typename U16Vec<CH>::type q = *reinterpret_cast<const typename U16Vec<CH>::type*>(
+            base + (leaf_off + row_pos<K>(x_at((uint32_t)c, D))));
+#pragma unroll
+        for (int u = 0; u < CH; ++u) cost[c + u] = f16_bits(q[u]);
+      }
+    }
+    uint32_t key[R];
+    levels<-1>(cost, key, edge, w);
+    // Lane 63 holds the minimum over every lane bit.
+    return reverse_digits((uint32_t)__builtin_amdgcn_readlane((int)key[0], 63) & NMASK);
+  }
 };
 
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+// Tree evaluation of a row that serves d + 1 steps, d < stride (the first
+// row of a walk; every later one serves a full stride).
+template <int K, int CB, int D>
+__device__ __forceinline__ uint32_t first_branches(int d, const uint16_t* row, uint32_t edge,
+                                                   const f16* w, int lane) {
+  static_assert(K * exl3::row_stride(K) <= 16 - K, "a row's branches fit in an edge");
+  if constexpr (D + 1 < exl3::row_stride(K)) {
+    if (d != D) return first_branches<K, CB, D + 1>(d, row, edge, w, lane);
+  }
+  return Tree<K, CB, D>(lane).branches(row, edge, w, -1);
 }
+
+// The walk of one tile by one wave. Row q of the walk (q = 0 .. rows - 1) is
+// stored row top - q * STRIDE and serves the steps above it down to the next
+// one. Each row's edge and branches are recorded (row q in lane q mod 64 of
+// a register, 64 rows at a time to LDS), and the states are rebuilt from the
+// records in parallel after the walk.
+template <int K, int CB>
+struct Walk {
+  static constexpr int KR = 16 - K, STRIDE = exl3::row_stride(K);
+  const Tree<K, CB, STRIDE - 1> tree;
+  const int lane, i_stop;
+  const f16* sw;      // inputs in step order
+  uint32_t* records;  // (branches << 16) | edge of each row
+  uint32_t rec = 0;
+  int i;              // the next step to decide
+  uint32_t edge;      // the edge reached after step i
+
+  __device__ __forceinline__ Walk(int lane_, int L, int i_stop_, uint32_t start, const f16* sw_,
+                                  uint32_t* records_)
+      : tree(lane_), lane(lane_), i_stop(i_stop_), sw(sw_), records(records_), i(L - 1),
+        edge((uint32_t)__builtin_amdgcn_readfirstlane((int)(start & ((65536u >> K) - 1u)))) {}
+
+  // Takes row q's first n branches: the newest digit goes on top of the edge.
+  __device__ __forceinline__ void take(int q, uint32_t ks, int n) {
+    if (lane == (q & 63)) rec = (ks << 16) | edge;
+    if ((q & 63) == 63) records[q - 63 + lane] = rec;
+    edge = ((ks & ((1u << (K * n)) - 1u)) << (KR - K * n)) | (edge >> (K * n));
+    i -= n;
+  }
+  __device__ __forceinline__ void first_row(const uint16_t* row) {
+    const int d = (i - 1) % STRIDE;
+    f16 w[STRIDE];
+#pragma unroll
+    for (int j = 0; j < STRIDE; ++j) w[j] = sw[i - j > 0 ? i - j : 0];
+    const int left = i - i_stop + 1;
+    take(0, first_branches<K, CB, 0>(d, row, edge, w, lane), left < d + 1 ? left : d + 1);
+  }
+  __device__ __forceinline__ uint32_t row_branches(const uint16_t* row) const {
+    f16 w[STRIDE];
+#pragma unroll
+    for (int j = 0; j < STRIDE; ++j) w[j] = sw[i - j];
+    return tree.branches(row, edge, w, -1);
+  }
+  __device__ __forceinline__ void next_row(int q, const uint16_t* row) {
+    take(q, row_branches(row), STRIDE);
+  }
+  // The walk's last row (of several), inside which it may end.
+  __device__ __forceinline__ void last_row(int q, const uint16_t* row) {
+    const int left = i - i_stop + 1;
+    take(q, row_branches(row), left < STRIDE ? left : STRIDE);
+  }
+  // Step 0, whose predecessors are the start constraint. Returns its state.
+  __device__ __forceinline__ uint32_t step0(int pre) {
+    const uint32_t k = Tree<K, CB, 0, true>(lane).branches(nullptr, edge, sw, pre);
+    const uint32_t sigma = (k << KR) | edge;
+    edge = sigma >> K;
+    return sigma;
+  }
+  // Sends the last records to LDS.
+  __device__ __forceinline__ void flush(int rows) {
+    const int q0 = (rows - 1) & ~63;
+    if (q0 + lane < rows) records[q0 + lane] = rec;
+  }
+  // State of step s >= 1 from the records.
+  __device__ __forceinline__ static uint32_t state(const uint32_t* records, int s, int L,
+                                                   int top) {
+    const int r0 = (s - 1) - (s - 1) % STRIDE;
+    const uint32_t rec = records[(top - r0) / STRIDE];
+    const int first = r0 + STRIDE < L - 1 ? r0 + STRIDE : L - 1;
+    const int n = first - s;  // branches of the row taken before step s
+    const uint32_t ks = rec >> 16, e = rec & 0xFFFFu;
+    const uint32_t at = ((ks & ((1u << (K * n)) - 1u)) << (KR - K * n)) | (e >> (K * n));
+    return (((ks >> (K * n)) & ((1u << K) - 1u)) << KR) | at;
+  }
+};
+
+// Copies the tile's fp16 inputs from its header to LDS in step order
+// (sw[i] = input (i + roll) mod L).
+__device__ __forceinline__ void load_step_inputs(const uint8_t* hdr, f16* sw, int L, int roll,
+                                                 int tid, int nt) {
+  const f16* src = reinterpret_cast<const f16*>(hdr + exl3::HDR_W_BYTES);
+  for (int r = tid; r < L; r += nt) sw[r >= roll ? r - roll : r - roll + L] = src[r];
+}
+
+// Steps the walk covers (its last step i_stop), the step of its first stored
+// row and its row count.
+template <int K>
+struct WalkSpan {
+  static constexpr int STRIDE = exl3::row_stride(K);
+  int i_stop, top, rows;
+  __device__ __forceinline__ explicit WalkSpan(const TbArgs& a) {
+    i_stop = a.write ? 0 : (a.L - a.roll) % a.L;
+    const int last_i = i_stop > 1 ? i_stop : 1;
+    top = (a.L - 2) - (a.L - 2) % STRIDE;
+    rows = (top - ((last_i - 1) - (last_i - 1) % STRIDE)) / STRIDE + 1;
+  }
+};
+
+// What a walk leaves: the states and their codebook values, coalesced over
+// the wave (write = 1), or the edge reached.
+template <int K, int CB>
+__device__ __forceinline__ void finish_walk(const TbArgs& a, int t, Walk<K, CB>& walk,
+                                            const WalkSpan<K>& span, int pre) {
+  const int lane = walk.lane;
+  const uint32_t sigma0 = span.i_stop == 0 ? walk.step0(pre) : 0u;
+  if (a.write) {
+    walk.flush(span.rows);
+    __builtin_amdgcn_wave_barrier();
+    for (int r = lane; r < a.L; r += 64) {
+      const int s = r >= a.roll ? r - a.roll : r - a.roll + a.L;
+      const uint32_t sigma = s == 0 ? sigma0 : Walk<K, CB>::state(walk.records, s, a.L, span.top);
+      a.out_idx[(int64_t)t * a.L + r] = (int16_t)(uint16_t)sigma;
+      a.out_w[(int64_t)t * a.L + r] = (float)decode_state(CB, sigma);
+    }
+  } else if (lane == 0) {
+    a.end_out[(int64_t)t * a.end_stride] = (int32_t)walk.edge;
+  }
+}
+
+// Per-row traceback: each stored row's tree is read straight from HBM, one
+// dependent load and one tree evaluation per row.
+template <int K, int CB>
+__global__ void __launch_bounds__(64) traceback_rows_kernel(TbArgs a) {
+  __shared__ f16 s_w[256];
+  __shared__ uint32_t s_record[256];
+  const int t = blockIdx.x;
+  const int lane = threadIdx.x;
+  const uint8_t* blk = a.scratch + (int64_t)t * a.tile_stride;
+  const uint8_t* hdr = blk + a.hdr_offset;
+  const int pre = reinterpret_cast<const int32_t*>(hdr)[exl3::HDR_PRE_STATE];
+  const uint32_t start = (uint32_t)a.start[(int64_t)t * a.start_stride];
+  load_step_inputs(hdr, s_w, a.L, a.roll, lane, 64);
+  __syncthreads();
+  const WalkSpan<K> span(a);
+  Walk<K, CB> walk(lane, a.L, span.i_stop, start, s_w, s_record);
+  const int row_elems = a.lay.row_bytes / 2;
+  const uint16_t* row = reinterpret_cast<const uint16_t*>(blk) +
+                        (int64_t)(span.top / Walk<K, CB>::STRIDE) * row_elems;
+  walk.first_row(row);
+  for (int q = 1; q < span.rows - 1; ++q) {
+    row -= row_elems;
+    walk.next_row(q, row);
+  }
+  if (span.rows > 1) walk.last_row(span.rows - 1, row - row_elems);
+  finish_walk<K, CB>(a, t, walk, span, pre);
+}
+
+// Streamed traceback for small batches. The per-row walk waits for one
+// dependent HBM load per stored row; with few tiles in flight that latency
+// is the whole kernel. The rows a walk visits are known in advance (only the
+// tree inside a row depends on the path), so here LOADERS waves copy whole
+// rows into an LDS ring ahead of the walk, straight from HBM to LDS
+// (global_load_lds, 16 bytes per lane), and wave 0 walks as above reading
+// its trees from the ring. A phase is G rows, one contiguous block of
+// scratch; the ring holds RING phases, of which one is walked while the
+// others are in flight, and there is one workgroup barrier per phase. It
+// reads every row whole (2E bytes instead of one tree), so it pays off only
+// while HBM bandwidth is idle.
+template <int K>
+struct StreamShape {
+  static constexpr int ROWB = 2 * (65536 >> K);
+  static constexpr int G = cmax((K <= 5 ? 16384 : (K <= 7 ? 8192 : 4096)) / ROWB, 1);
+  static constexpr int PHASE = G * ROWB;                // bytes per phase
+  static constexpr int RING = K == 1 || K >= 5 ? 2 : 3;
+  static constexpr int LOADERS = K <= 6 ? 4 : 1;
+  static constexpr int LOADS = PHASE / (LOADERS * 1024);  // per loader wave and phase
+  static constexpr int THREADS = 64 * (1 + LOADERS);
+  static_assert(LOADS * LOADERS * 1024 == PHASE, "a phase splits evenly over the loaders");
+  static_assert(LOADS * (RING - 1) <= 63, "the loads in flight fit in vmcnt");
+};
 
 template <int K, int CB>
 __global__ void __launch_bounds__(StreamShape<K>::THREADS) traceback_stream_kernel(TbArgs a) {
-  constexpr int KR = 16 - K;
-  constexpr int STRIDE = exl3::row_stride(K);
-  constexpr int RV = 2 * (65536 >> K) / 16;  // 16-byte vectors per row
-  constexpr int W = StreamShape<K>::W, NG = StreamShape<K>::NG;
-  constexpr int NLT = 64 * W;                // threads per loader group
-  // A row smaller than a loader group (K = 8: 32 vectors) leaves the
-  // group's threads lt >= RV idle.
-  constexpr bool PART = RV < NLT;
-  constexpr int V = PART ? 1 : RV / NLT;
-  static_assert(PART || RV % NLT == 0, "rows split evenly over a loader group");
-  __shared__ u32x4 s_ring[2][RV];
-  __shared__ uint16_t s_wbits[256];
-  __shared__ uint16_t s_oidx[256];
+  using S = StreamShape<K>;
+  __shared__ __attribute__((aligned(16))) uint8_t s_ring[S::RING][S::PHASE];
+  __shared__ f16 s_w[256];
+  __shared__ uint32_t s_record[256];
   const int t = blockIdx.x;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63;
-  const int L = a.L, roll = a.roll;
   const uint8_t* blk = a.scratch + (int64_t)t * a.tile_stride;
   const uint8_t* hdr = blk + a.hdr_offset;
-  const int row_bytes = a.lay.row_bytes;
+  const WalkSpan<K> span(a);
+  const int phases = (span.rows + S::G - 1) / S::G;
+  const int top_slot = span.top / exl3::row_stride(K);
+
+  if (wave > 0) {
+    // Phase p covers row slots top_slot - (p + 1) G + 1 .. top_slot - p G.
+    // Reads below the tile's first row (a last phase's rows that the walk
+    // does not visit, and phases past the last) are moved to that row.
+    auto issue = [&](int p) {
+      const int slot0 = top_slot - (p + 1) * S::G + 1;
+#pragma unroll
+      for (int j = 0; j < S::LOADS; ++j) {
+        const int piece = (j * S::LOADERS + wave - 1) * 1024;
+        const int off = slot0 * S::ROWB + piece + lane * 16;
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) void*)(blk + (off >= 0 ? off : lane * 16)),
+            (__attribute__((address_space(3))) void*)(&s_ring[p % S::RING][piece]), 16, 0, 0);
+      }
+    };
+#pragma unroll
+    for (int p = 0; p < S::RING - 1; ++p) issue(p);
+    for (int p = 0; p < phases; ++p) {
+      // Phase p has arrived (RING - 2 younger phases may be in flight), and
+      // past the barrier the walk has left phase p - 1's place in the ring.
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(S::LOADS * (S::RING - 2)) : "memory");
+      issue(p + S::RING - 1);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    return;
+  }
+
   const int pre = reinterpret_cast<const int32_t*>(hdr)[exl3::HDR_PRE_STATE];
-  const uint16_t* wsrc = reinterpret_cast<const uint16_t*>(hdr + exl3::HDR_W_BYTES);
-  for (int r = threadIdx.x; r < L; r += StreamShape<K>::THREADS) s_wbits[r] = wsrc[r];
-
-  // Steps L-1 .. i_stop are walked; steps >= 1 read the stored row
-  // r0(i) = (i - 1) - (i - 1) % STRIDE, rows top, top - STRIDE, ..., r_last.
-  const int i_stop = a.write ? 0 : (L - roll) % L;
-  const int last_i = i_stop > 1 ? i_stop : 1;
-  const int top = (L - 2) - (L - 2) % STRIDE;
-  const int r_last = (last_i - 1) - (last_i - 1) % STRIDE;
-  const int NR = (top - r_last) / STRIDE + 1;
-  auto row_src = [&](int q) {
-    return reinterpret_cast<const u32x4*>(blk + (int64_t)((top - q * STRIDE) / STRIDE) * row_bytes);
+  const uint32_t start = (uint32_t)a.start[(int64_t)t * a.start_stride];
+  load_step_inputs(hdr, s_w, a.L, a.roll, lane, 64);
+  Walk<K, CB> walk(lane, a.L, span.i_stop, start, s_w, s_record);
+  // Row q of the walk in the ring.
+  auto ring_row = [&](int q) {
+    const int p = q / S::G;
+    return reinterpret_cast<const uint16_t*>(s_ring[p % S::RING] +
+                                             (S::G - 1 - (q - p * S::G)) * S::ROWB);
   };
-
-  const int g = (wave - 1) / W;              // loader group (wave >= 1)
-  const int lt = threadIdx.x - 64 - g * NLT;
-  const bool loads = wave > 0 && (!PART || lt < RV);
-  u32x4 buf[V];  // native vectors: registers, not scratch
-  if (loads) {
-    if (g < NR) {
-      const u32x4* src = row_src(g);
-#pragma unroll
-      for (int v = 0; v < V; ++v) buf[v] = src[lt + v * NLT];
-    }
-    if (g == 0) {
-#pragma unroll
-      for (int v = 0; v < V; ++v) s_ring[0][lt + v * NLT] = buf[v];
-      if (NG < NR) {
-        const u32x4* src = row_src(NG);
-#pragma unroll
-        for (int v = 0; v < V; ++v) buf[v] = src[lt + v * NLT];
-      }
-    }
+  for (int p = 0; p < phases; ++p) {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    int q = p * S::G;
+    if (p == 0) walk.first_row(ring_row(q++));
+    const int q1 = cmin((p + 1) * S::G, span.rows - 1);
+    for (; q < q1; ++q) walk.next_row(q, ring_row(q));
   }
-  lds_barrier();
-
-  const uint16_t* wbits = s_wbits;
-  uint32_t edge = (uint32_t)a.start[(int64_t)t * a.start_stride] & ((65536u >> K) - 1u);
-  int i = L - 1;
-  for (int q = 0; q < NR; ++q) {
-    if (wave == 0) {
-      const uint16_t* row = reinterpret_cast<const uint16_t*>(s_ring[q & 1]);
-      const int r = top - q * STRIDE;
-      if (i >= last_i && (i - 1) - (i - 1) % STRIDE == r) {
-        // Steps i .. r + 1 read this row: one tree, one evaluation.
-        const int d = (i - 1) % STRIDE;
-        int ri = i + roll;
-        if (ri >= L) ri -= L;
-        const uint32_t ks = tb_tree_dispatch<K, CB, 0>(d, row, edge, wbits, ri, L, lane);
-#pragma unroll
-        for (int j = 0; j < STRIDE; ++j) {
-          if (j <= d && i >= last_i) {
-            int rj = i + roll;
-            if (rj >= L) rj -= L;
-            const uint32_t sigma = (((ks >> (K * j)) & ((1u << K) - 1u)) << KR) | edge;
-            if (a.write && lane == 0) s_oidx[rj] = (uint16_t)sigma;
-            edge = sigma >> K;
-            --i;
-          }
-        }
-      }
-    } else if (loads) {
-      const int j = q + 1;  // the row to place in the ring this iteration
-      if (j < NR && j % NG == g) {
-#pragma unroll
-        for (int v = 0; v < V; ++v) s_ring[j & 1][lt + v * NLT] = buf[v];
-        if (j + NG < NR) {
-          const u32x4* src = row_src(j + NG);
-#pragma unroll
-          for (int v = 0; v < V; ++v) buf[v] = src[lt + v * NLT];
-        }
-      }
-    }
-    lds_barrier();
-  }
-
-  if (wave != 0) return;
-  if (i_stop == 0) {  // step 0: predecessors from the start constraint
-    int ri = roll;
-    if (ri >= L) ri -= L;
-    const uint32_t k = tb_branch<K, CB, 0, true>(nullptr, edge, wbits, ri, L, lane, pre);
-    const uint32_t sigma = (k << KR) | edge;
-    if (a.write && lane == 0) s_oidx[ri] = (uint16_t)sigma;
-    edge = sigma >> K;
-  }
-  if (a.write) {
-    __builtin_amdgcn_wave_barrier();
-    for (int r = lane; r < L; r += 64) {
-      const uint32_t sigma = s_oidx[r];
-      a.out_idx[(int64_t)t * L + r] = (int16_t)(uint16_t)sigma;
-      a.out_w[(int64_t)t * L + r] = (float)decode_state(CB, sigma);
-    }
-  } else if (lane == 0) {
-    a.end_out[(int64_t)t * a.end_stride] = (int32_t)edge;
-  }
+  if (span.rows > 1) walk.last_row(span.rows - 1, ring_row(span.rows - 1));
+  finish_walk<K, CB>(a, t, walk, span, pre);
 }
 
 // ---------------------------------------------------------- prepare/finalize
@@ -1750,17 +1677,19 @@ static int resolve_policy(int policy) {
   return policy < 0 ? g_traceback_policy.load(std::memory_order_relaxed) : policy;
 }
 
-// The streamed traceback reads each visited row whole: per row it moves
-// tiles x row bytes at the streaming rate, where the per-row walk waits one
-// dependent tree load; the walk's row count cancels. Whole encode calls
-// measured the crossover at 128-256 tiles for K = 2, 3, about 384 for
-// K = 4, about 600 for K = 5 (each 2.5 MiB of rows per step of the walk)
-// and above 768 for K = 6..8, where the streamed kernel was 30-110 us per
-// call too long at 1024-2048 tiles.
+// The streamed traceback reads each visited row whole, so it is bound by the
+// bytes it streams, where the per-row walk waits for one dependent tree load
+// per row. Pass-1 + pass-2 tracebacks, streamed / per row: K = 4, 256 tiles
+// 77 / 87 us, 280 tiles 95 / 89; K = 5, 512 tiles 159 / 179, 560 tiles 190 /
+// 182; K = 6, 1024 tiles 166 / 194, 1200 tiles 206 / 201; K = 7, 2048 tiles
+// 165 / 218, 3000 tiles 300 / 246; K = 8, 4096 tiles 190 / 283: the line is
+// 2 MiB of rows per step of the walk. At K = 1..3, whose rows are 16 KiB and
+// more and serve 3 to 8 steps, the per-row walk is as fast from 16 tiles on
+// (K = 3: 49 / 56 us at 16 tiles, 49 / 65 at 64).
 static bool use_stream_traceback(const TbArgs& a, int policy) {
   if (policy == 1) return false;
   if (policy == 2) return true;
-  return (int64_t)a.n * a.lay.row_bytes <= ((int64_t)5 << 19) && a.n <= 768;
+  return a.lay.K >= 4 && (int64_t)a.n * a.lay.row_bytes <= ((int64_t)2 << 20);
 }
 
 template <int K>
