@@ -52,6 +52,9 @@ _SIGNATURES = {
     "exl3_hadamard128": (_c_int, [_c_vp, _c_vp, _c_i64, _c_i64, _c_int, _c_vp]),
     "exl3_hadamard128_scaled": (_c_int, [_c_vp, _c_vp, _c_i64, _c_i64, _c_int, _c_vp, _c_vp,
                                          _c_vp]),
+    "exl3_unrotate": (_c_int, [_c_vp, _c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_vp]),
+    "exl3_decode_weight": (_c_int, [_c_vp, _c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_int, _c_int,
+                                    _c_vp]),
     "exl3_block_rms_from_slices": (_c_int, [_c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_vp]),
     "exl3_block_rms": (_c_int, [_c_vp, _c_vp, _c_i64, _c_i64, _c_int, _c_int, _c_vp, _c_i64,
                                 _c_vp]),
@@ -518,6 +521,47 @@ def hadamard128_scaled(x, out, side: int, divisor=None, slice_sumsq=None) -> Non
             divisor.data_ptr() if divisor is not None else None,
             slice_sumsq.data_ptr() if slice_sumsq is not None else None, _stream(dev)),
             "hadamard128_scaled")
+
+
+def _scale_vector(t, name: str, numel: int, like) -> None:
+    torch = _torch()
+    if (not isinstance(t, torch.Tensor) or t.dtype != torch.float32 or not t.is_contiguous()
+            or t.device != like.device or t.numel() != numel):
+        raise RuntimeError(f"{name} must be a contiguous float32 tensor of {numel} elements on "
+                           f"{like.device}")
+
+
+def unrotate(x, su, sv, out) -> None:
+    """``out = (H x * su) H * sv`` with blockwise order-128 transforms
+    (exl3_unrotate); ``out`` must not be ``x``."""
+    dev = _matrix(x, "x")
+    _check_buffer(out, "out", x.dtype, tuple(x.shape), dev)
+    rows, cols = x.shape
+    _scale_vector(su, "su", rows, x)
+    _scale_vector(sv, "sv", cols, x)
+    torch = _torch()
+    with torch.cuda.device(dev):
+        _check(load_library().exl3_unrotate(x.data_ptr(), su.data_ptr(), sv.data_ptr(),
+                                            out.data_ptr(), rows, cols, _stream(dev)), "unrotate")
+
+
+def decode_weight(words, su, sv, out, K: int, cb: int) -> None:
+    """The (16 tk, 16 tn) weight of packed ``words`` ((tk * tn, 16 K) int16,
+    4-byte aligned) into ``out`` (exl3_decode_weight)."""
+    torch = _torch()
+    dev = _check_device_tensor(words, "words", torch.int16, 2)
+    _check_device_tensor(out, "out", torch.float32, 2)
+    rows, cols = out.shape
+    if words.shape[0] * 256 != rows * cols or words.shape[1] != 16 * K:
+        raise RuntimeError(f"words {tuple(words.shape)} do not hold a {rows} x {cols} weight at "
+                           f"K={K}")
+    _check_buffer(out, "out", torch.float32, (rows, cols), dev)
+    _scale_vector(su, "su", rows, out)
+    _scale_vector(sv, "sv", cols, out)
+    with torch.cuda.device(dev):
+        _check(load_library().exl3_decode_weight(words.data_ptr(), su.data_ptr(), sv.data_ptr(),
+                                                 out.data_ptr(), rows, cols, int(K), int(cb),
+                                                 _stream(dev)), "decode_weight")
 
 
 def block_rms_from_slices(slice_sumsq, out, n: int) -> None:

@@ -10,6 +10,9 @@
 //       levels 2..7 across lanes. Left (H @ x per 128-row block): one thread
 //       per column of a row block, the 128 values in registers; loads and
 //       stores are coalesced across the wave's 64 columns.
+//   unrotate_kernel
+//       the way back from the encoder's basis (both transforms and both
+//       scales) in one pass, from a matrix or straight from packed tiles.
 //   block_rms_slices_kernel / block_rms_reduce_kernel
 //       sqrt(sum of squares / n) along one dimension: one thread per slice
 //       of `blocksize` sums its squares in order, then one thread per output
@@ -31,6 +34,7 @@
 #include <stdint.h>
 
 #include "../../include/exl3_layer.h"
+#include "exl3_codebook.h"
 #include "exl3_errors.h"
 #include "exl3_layout.h"
 
@@ -126,6 +130,130 @@ __global__ void __launch_bounds__(256)
   }
 #pragma unroll
   for (int r = 0; r < HAD_N; ++r) out[base + r * cols] = v[r] * kHadScale;
+}
+
+// H_l, x su per row, H_r, x sv per column (hadamard.py:129-140) of one
+// 128 x 128 block per workgroup: the block is closed under both transforms,
+// so the whole way back is one read and one write of the matrix, where the
+// two transforms and two scalings by themselves are four of each. PACKED
+// reads the block's 64 tiles of stored trellis words instead of a matrix
+// (state, codebook value and tensor-core position computed in the kernel),
+// so a stored projection is decoded in one pass of K / 8 + 4 bytes per
+// weight. The fp32 operations and their order are those of the separate
+// passes: results are bit-identical to them.
+//
+// Eight waves. First half: wave w takes rows 32 (w / 2) .. + 31 of 64
+// columns, one column per lane, the 32 values in registers (butterfly
+// distances 1 .. 16), and leaves them in LDS. Second half: each wave takes
+// rows g, g + 32, g + 64, g + 96 (distances 32 and 64), two columns per
+// lane, scales them and transforms the four rows across the wave. 64 KiB of
+// LDS, two workgroups per CU. A 4096 x 4096 projection at K = 4 (75 MB)
+// decodes in 38 us; unpacking, a table lookup, the un-permutation, two
+// transforms and two scalings took 390 us.
+constexpr int UN_THREADS = 512;
+
+template <bool PACKED, int CB>
+__global__ void __launch_bounds__(UN_THREADS, 4)
+    unrotate_kernel(const float* __restrict__ in, const uint32_t* __restrict__ packed, int K,
+                    const float* __restrict__ su, const float* __restrict__ sv,
+                    float* __restrict__ out, int64_t cols) {
+  __shared__ __attribute__((aligned(16))) float s[HAD_N * HAD_N];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int half = wave & 1, r0 = (wave >> 1) * 32;
+  const int64_t row0 = (int64_t)blockIdx.y * HAD_N, col0 = (int64_t)blockIdx.x * HAD_N;
+
+  float v[32];
+  int c;  // the lane's column
+  if constexpr (PACKED) {
+    // Tile row `wave` of the block is 8 tiles, 64 K words, contiguous.
+    uint32_t* s_words = reinterpret_cast<uint32_t*>(s);
+    const uint32_t* src =
+        packed + ((row0 / 16 + wave) * (cols / 16) + col0 / 16) * (int64_t)(8 * K);
+    for (int j = 0; j < K; ++j) s_words[(wave * K + j) * 64 + lane] = src[j * 64 + lane];
+    __syncthreads();
+    // Column 8 half + lane % 8 of tile column lane / 8. Row 2 q + (e & 1) +
+    // 8 (e >> 1) of tile column cc + 8 half is encoded element i = 32 cc +
+    // 8 q + 4 half + e, whose state is the 16 bits of the tile's stream
+    // ending at bit (i + 1) K: the same bit offset in every lane, from word
+    // cc K on (a stored uint32 is 32 stream bits, most significant first).
+    const int cc = lane & 7, tc = lane >> 3;
+    c = tc * 16 + half * 8 + cc;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int tile = ((r0 / 16 + t) * 8 + tc) * 8 * K;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int last = (8 * q + 4 * half + e + 1) * K - 1;  // the window's last bit
+          const int word = cc * K + (last >> 5);
+          const uint32_t lo = s_words[tile + word];
+          const uint32_t hi = s_words[tile + (word > 0 ? word - 1 : 8 * K - 1)];
+          const uint32_t state = __builtin_amdgcn_alignbit(hi, lo, 31 - (last & 31)) & 0xFFFFu;
+          v[16 * t + 2 * q + (e & 1) + 8 * (e >> 1)] = (float)decode_state(CB, state);
+        }
+      }
+    }
+    __syncthreads();
+  } else {
+    c = half * 64 + lane;
+    const float* src = in + (row0 + r0) * cols + col0 + c;
+#pragma unroll
+    for (int r = 0; r < 32; ++r) v[r] = src[r * cols];
+  }
+#pragma unroll
+  for (int h = 1; h < 32; h <<= 1) {
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      if (!(i & h)) {
+        const float a = v[i], b = v[i + h];
+        v[i] = a + b;
+        v[i + h] = a - b;
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 32; ++r) s[(r0 + r) * HAD_N + c] = v[r];
+  __syncthreads();
+
+  const float2 d = reinterpret_cast<const float2*>(sv + col0)[lane];
+#pragma unroll 1
+  for (int g = wave; g < 32; g += 8) {
+    float2 x[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      x[j] = reinterpret_cast<const float2*>(s + (g + 32 * j) * HAD_N)[lane];
+#pragma unroll
+    for (int h = 1; h < 4; h <<= 1) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (!(j & h)) {
+          const float2 a = x[j], b = x[j + h];
+          x[j] = make_float2(a.x + b.x, a.y + b.y);
+          x[j + h] = make_float2(a.x - b.x, a.y - b.y);
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float u = su[row0 + g + 32 * j];
+      const float a = (x[j].x * kHadScale) * u, b = (x[j].y * kHadScale) * u;
+      x[j] = make_float2(a + b, a - b);
+    }
+#pragma unroll
+    for (int h = 1; h < 64; h <<= 1) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        x[j].x = had_level(x[j].x, lane, h);
+        x[j].y = had_level(x[j].y, lane, h);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      reinterpret_cast<float2*>(out + (row0 + g + 32 * j) * cols + col0)[lane] =
+          make_float2((x[j].x * kHadScale) * d.x, (x[j].y * kHadScale) * d.y);
+  }
 }
 
 // --------------------------------------------------------------- block RMS
@@ -358,6 +486,22 @@ int launch_hadamard(const float* in, float* out, int64_t rows, int64_t cols, int
   return check_launch(what);
 }
 
+// Checks and grid of the unrotate kernel: whole 128 x 128 blocks, out and sv
+// read and written as float2.
+int unrotate_grid(const void* in, const float* su, const float* sv, const float* out,
+                  int64_t rows, int64_t cols, dim3* grid, const char* what) {
+  if (!in || !su || !sv || !out) return set_error("%s: NULL buffer", what);
+  if (rows <= 0 || cols <= 0 || rows % HAD_N || cols % HAD_N)
+    return set_error("%s: both dimensions must be positive multiples of 128, got %lld x %lld",
+                     what, (long long)rows, (long long)cols);
+  if (((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(sv)) & 7) != 0)
+    return set_error("%s: out and sv must be 8-byte aligned", what);
+  if (cols / HAD_N > INT32_MAX || rows / HAD_N > 65535)
+    return set_error("%s: matrix too large", what);
+  *grid = dim3((unsigned)(cols / HAD_N), (unsigned)(rows / HAD_N));
+  return 0;
+}
+
 }  // namespace
 
 // ------------------------------------------------------------------- C-ABI
@@ -375,6 +519,36 @@ int exl3_hadamard128_scaled(const float* in, float* out, int64_t rows, int64_t c
     return set_error("hadamard128_scaled: slice sums of squares need side = 1");
   return launch_hadamard(in, out, rows, cols, side, divisor, slice_sumsq, stream,
                          "hadamard128_scaled");
+}
+
+int exl3_unrotate(const float* in, const float* su, const float* sv, float* out, int64_t rows,
+                  int64_t cols, void* stream) {
+  dim3 grid;
+  if (unrotate_grid(in, su, sv, out, rows, cols, &grid, "unrotate")) return 1;
+  hipLaunchKernelGGL((unrotate_kernel<false, 0>), grid, dim3(UN_THREADS), 0, as_stream(stream), in,
+                     nullptr, 0, su, sv, out, cols);
+  return check_launch("unrotate");
+}
+
+int exl3_decode_weight(const uint16_t* packed, const float* su, const float* sv, float* out,
+                       int64_t rows, int64_t cols, int K, int cb, void* stream) {
+  if (K < 1 || K > 8) return set_error("decode_weight: K must be in 1..8, got %d", K);
+  if (cb < 0 || cb > 2) return set_error("decode_weight: cb must be 0, 1, or 2, got %d", cb);
+  dim3 grid;
+  if (unrotate_grid(packed, su, sv, out, rows, cols, &grid, "decode_weight")) return 1;
+  if (reinterpret_cast<uintptr_t>(packed) & 3)
+    return set_error("decode_weight: the words must be 4-byte aligned");
+  const uint32_t* words = reinterpret_cast<const uint32_t*>(packed);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(UN_THREADS), 0, as_stream(stream), nullptr, words, K, su,
+                       sv, out, cols);
+  };
+  switch (cb) {
+    case 0: launch(unrotate_kernel<true, 0>); break;
+    case 1: launch(unrotate_kernel<true, 1>); break;
+    default: launch(unrotate_kernel<true, 2>); break;
+  }
+  return check_launch("decode_weight");
 }
 
 int exl3_block_rms_from_slices(const float* slice_sumsq, float* out, int64_t outputs, int64_t n,

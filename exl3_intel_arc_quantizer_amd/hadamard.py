@@ -53,20 +53,24 @@ def hadamard(n: int = HAD_DIM, dtype: torch.dtype = torch.float32,
     return _scaled_hadamard(n, dtype, factor, "cpu" if device is None else str(device))
 
 
-def _had128(x: torch.Tensor, side: int, had_dim: int, out: Optional[torch.Tensor]) -> torch.Tensor:
-    """The blockwise transform through the HIP fast Walsh-Hadamard kernel
-    (``exl3_hadamard128``); GPU tensors only."""
+def _check_blocks(x: torch.Tensor, sides: tuple, had_dim: int) -> None:
     if had_dim != HAD_DIM:
         raise ValueError(f"only had_dim={HAD_DIM} is supported, got {had_dim}")
     if x.dim() != 2:
         raise ValueError(f"expected a 2-D tensor, got shape {tuple(x.shape)}")
     k, n = x.shape
-    if side == 0 and k % had_dim != 0:
+    if 0 in sides and k % had_dim != 0:
         raise ValueError(f"rows ({k}) must be divisible by had_dim ({had_dim})")
-    if side == 1 and n % had_dim != 0:
+    if 1 in sides and n % had_dim != 0:
         raise ValueError(f"columns ({n}) must be divisible by had_dim ({had_dim})")
     if x.device.type != "cuda":
         raise ValueError("the Hadamard transforms run on the GPU; move the tensor to a cuda device")
+
+
+def _had128(x: torch.Tensor, side: int, had_dim: int, out: Optional[torch.Tensor]) -> torch.Tensor:
+    """The blockwise transform through the HIP fast Walsh-Hadamard kernel
+    (``exl3_hadamard128``); GPU tensors only."""
+    _check_blocks(x, (side,), had_dim)
     from ._native import hadamard128
     work = x if (x.dtype == torch.float32 and x.is_contiguous()) else \
         x.to(torch.float32).contiguous()
@@ -108,14 +112,28 @@ def blockwise_preapply_had_r_(x: torch.Tensor, had_dim: int = HAD_DIM) -> torch.
     return _in_place(x, 1, had_dim)
 
 
+def scale_vectors(su: torch.Tensor, sv: torch.Tensor, k: int, n: int,
+                  device: torch.device) -> tuple:
+    """su and sv as float32 vectors on ``device``, sv 8-byte aligned."""
+    if su.numel() != k or sv.numel() != n:
+        raise ValueError(f"su must have {k} elements and sv {n}, got {su.numel()} / {sv.numel()}")
+    su = su.to(device=device, dtype=torch.float32).reshape(k).contiguous()
+    sv = sv.to(device=device, dtype=torch.float32).reshape(n).contiguous()
+    return su, (sv.clone() if sv.data_ptr() % 8 else sv)
+
+
 def weight_from_quantized(w_hat: torch.Tensor, su: torch.Tensor,
                           sv: torch.Tensor) -> torch.Tensor:
     """Original-basis weight from the transformed reconstruction: H_l, x su,
-    H_r, x sv (hadamard.py:129-140)."""
+    H_r, x sv (hadamard.py:129-140), a new float32 tensor. One pass over HBM
+    (``exl3_unrotate``)."""
     k, n = w_hat.shape
     if su.numel() != k or sv.numel() != n:
         raise ValueError(f"su must have {k} elements and sv {n}, got {su.numel()} / {sv.numel()}")
-    work = _had128(w_hat, 0, HAD_DIM, None)          # a new tensor: w_hat is not modified
-    work.mul_(su.to(device=work.device, dtype=torch.float32).reshape(k, 1))
-    _had128(work, 1, HAD_DIM, work)
-    return work.mul_(sv.to(device=work.device, dtype=torch.float32).reshape(1, n))
+    _check_blocks(w_hat, (0, 1), HAD_DIM)
+    from ._native import unrotate
+    work = w_hat if (w_hat.dtype == torch.float32 and w_hat.is_contiguous()) else \
+        w_hat.to(torch.float32).contiguous()
+    out = torch.empty_like(work)
+    unrotate(work, *scale_vectors(su, sv, k, n, work.device), out)
+    return out

@@ -21,8 +21,8 @@ from typing import Any, Dict, Optional, Tuple, Union
 
 import torch
 
-from .hadamard import weight_from_quantized
-from .trellis_format import CB_3INST, CB_MCG, CB_MUL1, tensor_core_perm
+from .hadamard import HAD_DIM, scale_vectors
+from .trellis_format import CB_3INST, CB_MCG, CB_MUL1
 
 __all__ = ["pack_module_trellis", "unpack_module_trellis", "decode_weight_from_storage",
            "build_layer_tensors", "export_layer_safetensors", "load_and_verify_layer_safetensors"]
@@ -83,20 +83,21 @@ def decode_weight_from_storage(trellis: torch.Tensor, suh: torch.Tensor, svh: to
                                K: int, cb: int = CB_MUL1) -> torch.Tensor:
     """Original-basis (k, n) float32 weight from stored EXL3 tensors
     (serialization.py:223-266): unpack, codebook values, tiles back to their
-    original element order, then Hadamard and scales. On the trellis'
-    device."""
-    tk, tn, _ = trellis.shape
-    dev_trellis = _on_gpu(trellis)
-    device = dev_trellis.device
-    states = unpack_module_trellis(dev_trellis, K).to(torch.int64) & 0xFFFF
-    lut = torch.empty(65536, dtype=torch.float16, device=device)
-    _ext().decode_codebook(cb, lut)
-    vals = lut[states].to(torch.float32)                                  # (tk, tn, 256) TC order
-    perm = torch.as_tensor(tensor_core_perm(), dtype=torch.long, device=device)
-    tiles = torch.empty_like(vals)
-    tiles[..., perm] = vals
-    w_hat = tiles.view(tk, tn, 16, 16).permute(0, 2, 1, 3).reshape(tk * 16, tn * 16)
-    w = weight_from_quantized(w_hat, suh.to(device).unsqueeze(1), svh.to(device).unsqueeze(0))
+    original element order, then Hadamard and scales, in one pass
+    (``exl3_decode_weight``). On the trellis' device."""
+    tk, tn, words = trellis.shape
+    k, n = tk * 16, tn * 16
+    if words != 16 * K:
+        raise ValueError(f"Trellis last dimension {words} does not match 16 * K = {16 * K}")
+    if k % HAD_DIM or n % HAD_DIM:
+        raise ValueError(f"both dimensions must be divisible by {HAD_DIM}, got {(k, n)}")
+    from ._native import decode_weight
+    packed = _on_gpu(trellis).to(torch.int16).reshape(tk * tn, words).contiguous()
+    if packed.data_ptr() % 4:
+        packed = packed.clone()
+    su, sv = scale_vectors(suh, svh, k, n, packed.device)
+    w = torch.empty((k, n), dtype=torch.float32, device=packed.device)
+    decode_weight(packed, su, sv, w, K, cb)
     return w.to(trellis.device)
 
 

@@ -41,6 +41,21 @@ int exl3_hadamard128(const float* in, float* out, int64_t rows, int64_t cols, in
 int exl3_hadamard128_scaled(const float* in, float* out, int64_t rows, int64_t cols, int side,
                             const float* divisor, float* slice_sumsq, void* stream);
 
+/* Replaces weight_from_quantized (hadamard.py:129-140): out = (H (in) * su)
+ * H * sv with the blockwise transforms of exl3_hadamard128, su of `rows`
+ * floats (one per row), sv of `cols` floats, in one pass over HBM; the same
+ * fp32 operations as the separate transforms and scalings. rows and cols are
+ * multiples of 128; out and sv are 8-byte aligned; out does not overlap in. */
+int exl3_unrotate(const float* in, const float* su, const float* sv, float* out, int64_t rows,
+                  int64_t cols, void* stream);
+
+/* Replaces decode_weight_from_storage (serialization.py:223-266): the weight
+ * of a stored projection, exl3_unrotate of the codebook values of its packed
+ * tiles (uint16 [rows / 16][cols / 16][16 K], the words exl3_pack_trellis
+ * writes, 4-byte aligned) with codebook cb, in one pass. */
+int exl3_decode_weight(const uint16_t* packed, const float* su, const float* sv, float* out,
+                       int64_t rows, int64_t cols, int K, int cb, void* stream);
+
 /* Second pass of block_rms (regularize.py:41-56) over slice sums made
  * elsewhere: out[o] = sqrt(S_o / n), S_o the sum of slice_sumsq[o * slices
  * + s] over s = 0 .. slices - 1 taken in slice order. */
