@@ -56,6 +56,9 @@ _SIGNATURES = {
     "exl3_decode_weight": (_c_int, [_c_vp, _c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_int, _c_int,
                                     _c_vp]),
     "exl3_block_rms_from_slices": (_c_int, [_c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_vp]),
+    "exl3_input_scales": (_c_int, [_c_vp, _c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_vp]),
+    "exl3_output_scales": (_c_int, [_c_vp, _c_i64, _c_i64, _c_vp, _c_i64, _c_i64, _c_vp, _c_int,
+                                    _c_int, _c_vp, _c_i64, _c_vp, _c_vp, _c_vp, _c_vp, _c_vp]),
     "exl3_block_rms": (_c_int, [_c_vp, _c_vp, _c_i64, _c_i64, _c_int, _c_int, _c_vp, _c_i64,
                                 _c_vp]),
     "exl3_block_rms_workspace": (_c_i64, [_c_i64, _c_i64, _c_int, _c_int]),
@@ -577,6 +580,46 @@ def block_rms_from_slices(slice_sumsq, out, n: int) -> None:
         _check(load_library().exl3_block_rms_from_slices(slice_sumsq.data_ptr(), out.data_ptr(),
                                                          outputs, int(n), slices, _stream(dev)),
                "block_rms_from_slices")
+
+
+def input_scales(slice_sumsq, su, scales, su_out, n: int) -> None:
+    """regularize's input-channel scales and su from the slice sums of
+    squares of (rows, n) (exl3_input_scales)."""
+    torch = _torch()
+    dev = _matrix(slice_sumsq, "slice_sumsq")
+    rows, slices = slice_sumsq.shape
+    for t, name in ((su, "su"), (scales, "scales"), (su_out, "su_out")):
+        _scale_vector(t, name, rows, slice_sumsq)
+    with torch.cuda.device(dev):
+        _check(load_library().exl3_input_scales(slice_sumsq.data_ptr(), su.data_ptr(),
+                                                scales.data_ptr(), su_out.data_ptr(), rows,
+                                                int(n), slices, _stream(dev)), "input_scales")
+
+
+def output_scales(x, sv, decide: int, forced: bool, scales, divisor, sv_out, flags,
+                  diag=None) -> None:
+    """regularize's output-channel scales (exl3_output_scales). ``diag`` is a
+    1-D float32 tensor on x's device, of any positive stride."""
+    torch = _torch()
+    dev = _matrix(x, "x")
+    rows, cols = x.shape
+    for t, name in ((sv, "sv"), (scales, "scales"), (divisor, "divisor"), (sv_out, "sv_out")):
+        _scale_vector(t, name, cols, x)
+    _check_buffer(flags, "flags", torch.float64, (3,), dev)
+    if diag is not None and (diag.dtype != torch.float32 or diag.dim() != 1
+                             or diag.device != x.device or diag.numel() < 1
+                             or diag.stride(0) < 1):
+        raise RuntimeError(f"diag must be a 1-D float32 tensor on {x.device}, not expanded")
+    lib = load_library()
+    with torch.cuda.device(dev):
+        need = int(lib.exl3_block_rms_workspace(rows, cols, 0, 32))
+        ws = torch.empty(max(need, 1), dtype=torch.float32, device=x.device)
+        _check(lib.exl3_output_scales(
+            x.data_ptr(), rows, cols, diag.data_ptr() if diag is not None else None,
+            diag.stride(0) if diag is not None else 1,
+            diag.numel() if diag is not None else 0, sv.data_ptr(), int(decide),
+            int(bool(forced)), ws.data_ptr(), ws.numel(), scales.data_ptr(), divisor.data_ptr(),
+            sv_out.data_ptr(), flags.data_ptr(), _stream(dev)), "output_scales")
 
 
 def block_rms(x, out, dim: int, blocksize: int = 32) -> None:

@@ -13,10 +13,13 @@
 //   unrotate_kernel
 //       the way back from the encoder's basis (both transforms and both
 //       scales) in one pass, from a matrix or straight from packed tiles.
-//   block_rms_slices_kernel / block_rms_reduce_kernel
+//   block_rms_slices_kernel / block_rms_reduce_{columns,rows}_kernel
 //       sqrt(sum of squares / n) along one dimension: one thread per slice
 //       of `blocksize` sums its squares in order, then one thread per output
 //       accumulates the slice sums in slice order.
+//   column_scales_kernel / output_scales_kernel
+//       regularize's output-channel scales from the column slice sums, with
+//       the skew decision on the device.
 //   cholesky_diag_kernel
 //       the unblocked Cholesky factorisation of one diagonal block (order
 //       <= 128) inside a blocked factorisation whose panel updates and
@@ -282,17 +285,223 @@ __global__ void __launch_bounds__(256)
 }
 
 // Pass 2: one thread per output accumulates its slice sums in slice order.
-__global__ void __launch_bounds__(256)
-    block_rms_reduce_kernel(const float* __restrict__ ws, float* __restrict__ out,
-                            int64_t outputs, int64_t n, int64_t ns, int dim) {
-  const int64_t o = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (o >= outputs) return;
+// The additions are one dependent chain, the loads are not: RMS_BATCH of
+// them are issued together, so a chain of 128 slices waits for memory 4
+// times instead of 128 (4096 outputs, 128 slices: 18.7 us one load at a
+// time).
+constexpr int RMS_BATCH = 32;
+
+template <class Load>
+__device__ __forceinline__ float ordered_sum(int64_t ns, Load load) {
   float acc = 0.0f;
-  for (int64_t s = 0; s < ns; ++s) {
-    const float v = dim == 0 ? ws[s * outputs + o] : ws[o * ns + s];
+  int64_t s = 0;
+  for (; s + RMS_BATCH <= ns; s += RMS_BATCH) {
+    float v[RMS_BATCH];
+#pragma unroll
+    for (int j = 0; j < RMS_BATCH; ++j) v[j] = load(s + j);
+#pragma unroll
+    for (int j = 0; j < RMS_BATCH; ++j) acc = (s + j == 0) ? v[j] : acc + v[j];
+  }
+  for (; s < ns; ++s) {
+    const float v = load(s);
     acc = (s == 0) ? v : acc + v;
   }
-  out[o] = sqrtf(acc / (float)n);
+  return acc;
+}
+
+// dim = 0: ws[s * outputs + o], coalesced over the outputs.
+__global__ void __launch_bounds__(64)
+    block_rms_reduce_columns_kernel(const float* __restrict__ ws, float* __restrict__ out,
+                                    int64_t outputs, int64_t n, int64_t ns) {
+  const int64_t o = (int64_t)blockIdx.x * 64 + threadIdx.x;
+  if (o >= outputs) return;
+  out[o] = sqrtf(ordered_sum(ns, [&](int64_t s) { return ws[s * outputs + o]; }) / (float)n);
+}
+
+// dim = 1: ws[o * ns + s]. A workgroup's ROWS_RED outputs are contiguous in
+// ws, so their slice sums pass through LDS in chunks of ROWS_CHUNK, loaded
+// along the rows (coalesced) and summed down them by one lane per output
+// (a row stride of ROWS_CHUNK + 1: 64 different banks). 4096 outputs, 128
+// slices: 37.6 us with strided loads from HBM, 4.0 us here.
+// su != NULL: the output is an input-channel scale and the row's sign-folded
+// divisor goes to su_out (regularize.py:171-181): a scale that is zero
+// becomes 0.1, su_out = su * scale / -1.24371088 + 1e-10, where the division
+// by the constant is a multiplication by its reciprocal, as torch divides by
+// a host scalar.
+constexpr int ROWS_RED = 64, ROWS_CHUNK = 128;
+
+constexpr float kTiny = 1e-30f;       // below this an RMS counts as zero
+constexpr float kZeroFloor = 0.1f;    // scale of an all-zero row or column
+constexpr float kScaleEps = 1e-10f;   // added to every scale
+constexpr float kCodebookScale = 1.24371088f;
+constexpr float kSkewCutoff = 0.15f;  // output scales only below this skew
+constexpr int kSkewFraction = 50;     // the skew looks at the top 1/50 of the diagonal
+
+__global__ void __launch_bounds__(256)
+    block_rms_reduce_rows_kernel(const float* __restrict__ ws, float* __restrict__ out,
+                                 int64_t outputs, int64_t n, int64_t ns,
+                                 const float* __restrict__ su, float* __restrict__ su_out) {
+  __shared__ float s_v[ROWS_RED][ROWS_CHUNK + 1];
+  const int64_t o0 = (int64_t)blockIdx.x * ROWS_RED;
+  const int rows = outputs - o0 < ROWS_RED ? (int)(outputs - o0) : ROWS_RED;
+  float acc = 0.0f;
+  for (int64_t s0 = 0; s0 < ns; s0 += ROWS_CHUNK) {
+    const int len = ns - s0 < ROWS_CHUNK ? (int)(ns - s0) : ROWS_CHUNK;
+#pragma unroll 8
+    for (int i = threadIdx.x; i < rows * ROWS_CHUNK; i += 256) {
+      const int r = i / ROWS_CHUNK, c = i % ROWS_CHUNK;
+      if (c < len) s_v[r][c] = ws[(o0 + r) * ns + s0 + c];
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < rows) {
+      const float* row = s_v[threadIdx.x];
+      const float part = ordered_sum(len, [&](int64_t c) {
+        return c == 0 && s0 > 0 ? acc + row[0] : row[c];
+      });
+      acc = part;
+    }
+    __syncthreads();
+  }
+  if ((int)threadIdx.x >= rows) return;
+  const int64_t o = o0 + threadIdx.x;
+  float v = sqrtf(acc / (float)n);
+  if (su != nullptr) {
+    if (fabsf(v) < kTiny) v = kZeroFloor;
+    su_out[o] = (su[o] * v) * (1.0f / -kCodebookScale) + kScaleEps;
+  }
+  out[o] = v;
+}
+
+// ----------------------------------------------------------- output scales
+
+constexpr int SC_THREADS = 1024;
+
+// Sum over the workgroup, in every thread.
+__device__ __forceinline__ double block_sum(double v, double* s_red) {
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double t = 0.0;
+  for (int w = 0; w < SC_THREADS / 64; ++w) t += s_red[w];
+  return t;
+}
+
+// Share of sum(sqrt(diag)) held by its largest len / 50 entries
+// (regularize.py:102-118), by one workgroup: the m-th largest value is found
+// by radix selection over the bits of the (non-negative) roots, eight bits a
+// pass, so nothing is sorted. Sums in double. A NaN root makes the skew NaN.
+__device__ float diagonal_skew(const float* __restrict__ diag, int64_t stride, int64_t len,
+                               uint32_t* s_hist, uint32_t* s_pick, double* s_red) {
+  const int64_t m = len / kSkewFraction;
+  auto root = [&](int64_t i) { return sqrtf(diag[i * stride]) + 0.0f; };
+  uint32_t prefix = 0, left = (uint32_t)m;
+  for (int shift = 24; m > 0 && shift >= 0; shift -= 8) {
+    for (int b = threadIdx.x; b < 256; b += SC_THREADS) s_hist[b] = 0;
+    __syncthreads();
+    for (int64_t i = threadIdx.x; i < len; i += SC_THREADS) {
+      const uint32_t bits = __float_as_uint(root(i));
+      if (shift == 24 || (bits >> (shift + 8)) == prefix)
+        atomicAdd(&s_hist[(bits >> shift) & 255u], 1u);
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {
+      // Lane l holds bins 255 - 4 l .. 252 - 4 l; the bin where the count
+      // from the top reaches `left` is the next byte.
+      const int lane = threadIdx.x;
+      uint32_t c[4], own = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) own += c[j] = s_hist[255 - 4 * lane - j];
+      uint32_t upto = own;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_up((int)upto, d, 64);
+        if (lane >= d) upto += o;
+      }
+      uint32_t before = upto - own;
+      if (before < left && upto >= left) {
+        int j = 0;
+        while (before + c[j] < left) before += c[j++];
+        s_pick[0] = (prefix << 8) | (uint32_t)(255 - 4 * lane - j);
+        s_pick[1] = left - before;
+      }
+    }
+    __syncthreads();
+    prefix = s_pick[0];
+    left = s_pick[1];
+    __syncthreads();
+  }
+  double all = 0.0, top = 0.0;
+  for (int64_t i = threadIdx.x; i < len; i += SC_THREADS) {
+    const float r = root(i);
+    all += (double)r;
+    if (m > 0 && __float_as_uint(r) > prefix) top += (double)r;
+  }
+  all = block_sum(all, s_red);
+  top = block_sum(top, s_red);
+  if (m > 0) top += (double)left * (double)__uint_as_float(prefix);
+  // A NaN root is in `all`; the quotient is NaN whatever was selected.
+  return (float)top / (float)all;
+}
+
+// Column RMS from the slice sums, and (one more workgroup, beside them) the
+// skew of the Hessian diagonal into flags[1].
+__global__ void __launch_bounds__(SC_THREADS)
+    column_scales_kernel(const float* __restrict__ ws, float* __restrict__ scales, int64_t cols,
+                         int64_t rows, int64_t ns, const float* __restrict__ diag,
+                         int64_t diag_stride, int64_t diag_len, double* __restrict__ flags) {
+  __shared__ uint32_t s_hist[256];
+  __shared__ uint32_t s_pick[2];
+  __shared__ double s_red[SC_THREADS / 64];
+  // Columns are taken 64 to a wave, the workgroup's first wave only: the
+  // launch has one workgroup per 64 columns.
+  if ((int64_t)blockIdx.x * 64 < cols) {
+    const int64_t o = (int64_t)blockIdx.x * 64 + threadIdx.x;
+    if (threadIdx.x < 64 && o < cols)
+      scales[o] =
+          sqrtf(ordered_sum(ns, [&](int64_t s) { return ws[s * cols + o]; }) / (float)rows);
+    return;
+  }
+  const float skew = diagonal_skew(diag, diag_stride, diag_len, s_hist, s_pick, s_red);
+  if (threadIdx.x == 0) flags[1] = (double)skew;
+}
+
+// The output-channel scales of regularize (regularize.py:136-168) from the
+// column RMS, in one workgroup: normalised by their mean unless W has no
+// energy, zero columns floored and sv folded where the scales apply. decide:
+// 0 never, 1 always, 2 where the skew (flags[1]) is below the cutoff; forced:
+// they also apply where W has no energy. divisor is what W's columns are
+// divided by, sv_out the same with zeros for the dead columns. flags =
+// {any energy, skew, applied}.
+__global__ void __launch_bounds__(SC_THREADS)
+    output_scales_kernel(float* __restrict__ scales, int64_t cols,
+                         const float* __restrict__ sv, int decide, int forced,
+                         float* __restrict__ divisor, float* __restrict__ sv_out,
+                         double* __restrict__ flags) {
+  __shared__ double s_red[SC_THREADS / 64];
+  double sum = 0.0;
+  for (int64_t i = threadIdx.x; i < cols; i += SC_THREADS) sum += (double)scales[i];
+  const float mean = (float)(block_sum(sum, s_red) / (double)cols);
+  const bool live = mean > kTiny;
+  const bool apply = (forced && !live) || decide == 1 ||
+                     (decide == 2 && (float)flags[1] < kSkewCutoff);
+  for (int64_t i = threadIdx.x; i < cols; i += SC_THREADS) {
+    float v = scales[i] / (live ? mean : 1.0f);
+    const bool dead = fabsf(v) < kTiny;
+    float d = sv[i];
+    if (apply) {
+      if (dead) v = kZeroFloor;
+      d = d * v + kScaleEps;
+    }
+    scales[i] = v;
+    divisor[i] = d;
+    sv_out[i] = dead ? 0.0f : d;
+  }
+  if (threadIdx.x == 0) {
+    flags[0] = live ? 1.0 : 0.0;
+    flags[2] = apply ? 1.0 : 0.0;
+  }
 }
 
 // -------------------------------------------------------- Cholesky block
@@ -558,10 +767,52 @@ int exl3_block_rms_from_slices(const float* slice_sumsq, float* out, int64_t out
     return set_error("block_rms_from_slices: empty shape (%lld outputs, n %lld, %lld slices)",
                      (long long)outputs, (long long)n, (long long)slices);
   unsigned b;
-  if (exl3::grid_1d(outputs, 256, &b, "block_rms_from_slices")) return 1;
-  hipLaunchKernelGGL(block_rms_reduce_kernel, dim3(b), dim3(256), 0, as_stream(stream),
-                     slice_sumsq, out, outputs, n, slices, 1);
+  if (exl3::grid_1d(outputs, ROWS_RED, &b, "block_rms_from_slices")) return 1;
+  hipLaunchKernelGGL(block_rms_reduce_rows_kernel, dim3(b), dim3(256), 0, as_stream(stream),
+                     slice_sumsq, out, outputs, n, slices, nullptr, nullptr);
   return check_launch("block_rms_from_slices");
+}
+
+int exl3_input_scales(const float* slice_sumsq, const float* su, float* scales, float* su_out,
+                      int64_t rows, int64_t n, int64_t slices, void* stream) {
+  if (!slice_sumsq || !su || !scales || !su_out) return set_error("input_scales: NULL buffer");
+  if (rows <= 0 || n <= 0 || slices <= 0)
+    return set_error("input_scales: empty shape (%lld rows, n %lld, %lld slices)",
+                     (long long)rows, (long long)n, (long long)slices);
+  unsigned b;
+  if (exl3::grid_1d(rows, ROWS_RED, &b, "input_scales")) return 1;
+  hipLaunchKernelGGL(block_rms_reduce_rows_kernel, dim3(b), dim3(256), 0, as_stream(stream),
+                     slice_sumsq, scales, rows, n, slices, su, su_out);
+  return check_launch("input_scales");
+}
+
+int exl3_output_scales(const float* x, int64_t rows, int64_t cols, const float* diag,
+                       int64_t diag_stride, int64_t diag_len, const float* sv, int decide,
+                       int forced, float* workspace, int64_t workspace_elems, float* scales,
+                       float* divisor, float* sv_out, double* flags, void* stream) {
+  constexpr int bs = 32;
+  if (!x || !sv || !workspace || !scales || !divisor || !sv_out || !flags)
+    return set_error("output_scales: NULL buffer");
+  if (rows <= 0 || cols <= 0) return set_error("output_scales: empty matrix");
+  if (decide < 0 || decide > 2) return set_error("output_scales: decide must be 0, 1 or 2");
+  if (diag && (diag_len <= 0 || diag_len > INT32_MAX || diag_stride < 1))
+    return set_error("output_scales: bad diagonal (%lld values, stride %lld)",
+                     (long long)diag_len, (long long)diag_stride);
+  const int64_t ns = (rows + bs - 1) / bs;
+  if (workspace_elems < cols * ns)
+    return set_error("output_scales: workspace holds %lld floats, %lld needed",
+                     (long long)workspace_elems, (long long)(cols * ns));
+  unsigned b1, b2;
+  if (exl3::grid_1d(cols * ns, 256, &b1, "output_scales")) return 1;
+  if (exl3::grid_1d(cols, 64, &b2, "output_scales")) return 1;
+  hipStream_t sm = as_stream(stream);
+  hipLaunchKernelGGL(block_rms_slices_kernel, dim3(b1), dim3(256), 0, sm, x, workspace, cols,
+                     rows, 1, cols, bs, ns, 0);
+  hipLaunchKernelGGL(column_scales_kernel, dim3(b2 + (diag ? 1 : 0)), dim3(SC_THREADS), 0, sm,
+                     workspace, scales, cols, rows, ns, diag, diag_stride, diag_len, flags);
+  hipLaunchKernelGGL(output_scales_kernel, dim3(1), dim3(SC_THREADS), 0, sm, scales, cols, sv,
+                     decide, forced, divisor, sv_out, flags);
+  return check_launch("output_scales");
 }
 
 int64_t exl3_block_rms_workspace(int64_t rows, int64_t cols, int dim, int blocksize) {
@@ -586,13 +837,18 @@ int exl3_block_rms(const float* x, float* out, int64_t rows, int64_t cols, int d
   const int64_t ns = (n + blocksize - 1) / blocksize;
   unsigned b1, b2;
   if (exl3::grid_1d(outputs * ns, 256, &b1, "block_rms")) return 1;
-  if (exl3::grid_1d(outputs, 256, &b2, "block_rms")) return 1;
+  if (exl3::grid_1d(outputs, 64, &b2, "block_rms")) return 1;
+  static_assert(ROWS_RED == 64, "both reductions take 64 outputs to a workgroup");
   hipStream_t sm = as_stream(stream);
   hipLaunchKernelGGL(block_rms_slices_kernel, dim3(b1), dim3(256), 0, sm, x, workspace, outputs, n,
                      so, st, blocksize, ns, dim);
   if (check_launch("block_rms")) return 1;
-  hipLaunchKernelGGL(block_rms_reduce_kernel, dim3(b2), dim3(256), 0, sm, workspace, out, outputs,
-                     n, ns, dim);
+  if (dim == 0)
+    hipLaunchKernelGGL(block_rms_reduce_columns_kernel, dim3(b2), dim3(64), 0, sm, workspace, out,
+                       outputs, n, ns);
+  else
+    hipLaunchKernelGGL(block_rms_reduce_rows_kernel, dim3(b2), dim3(256), 0, sm, workspace, out,
+                       outputs, n, ns, nullptr, nullptr);
   return check_launch("block_rms");
 }
 

@@ -19,17 +19,20 @@ How it runs here. The reference spends about a dozen full passes over the
 matrix (clone, RMS, division, transform, RMS, division, transform). This
 module makes three, on HIP kernels of ``libexl3_hip.so``:
 
-1. ``exl3_block_rms`` along the columns of W (two launches);
+1. ``exl3_output_scales``: the column RMS of W, its mean, the skew of the
+   Hessian diagonal (radix selection of its largest 2 %) and sv, every
+   decision taken on the device;
 2. ``exl3_hadamard128_scaled`` side 1: W / sv and the right transform into a
    new matrix in one read and one write, with the sums of squares of every
-   32-element row slice as a by-product; ``exl3_block_rms_from_slices``
-   turns those into the row RMS (a reduction over k x n/32 floats);
+   32-element row slice as a by-product; ``exl3_input_scales`` turns those
+   into the row RMS and su (a reduction over k x n/32 floats);
 3. ``exl3_hadamard128_scaled`` side 0: division by su and the left
    transform, in place.
 
-The scale vectors (n and k floats) are handled by torch between the passes;
-one host read of the mean column RMS decides the all-zero case, as in the
-reference.
+The decisions (any energy, skew, scales applied) come back in one read after
+the last pass. A 4096 x 4096 weight takes 140 us, where torch operations on
+the scale vectors between the passes, a sort of the diagonal and strided
+reductions took 322 us.
 
 Rounding. Divisions are correctly rounded fp32, like torch's; the transform
 is the fast Walsh-Hadamard transform of ``exl3_hadamard128``. The RMS splits
@@ -49,6 +52,7 @@ import torch
 
 from .hadamard import HAD_DIM
 
+# The kernels of exl3_output_scales / exl3_input_scales carry these values.
 CODEBOOK_SCALE = 1.24371088     # the codebook's RMS, regularize.py:33
 OUT_SCALE_SKEW_CUTOFF = 0.15    # output scales only below this skew
 SKEW_FRACTION = 50              # the skew looks at the top 1/50 of the diagonal
@@ -107,17 +111,17 @@ def hessian_skew(H_diag: torch.Tensor) -> float:
 
 
 def _out_scale_decision(H_diag: Optional[torch.Tensor], forced: Optional[bool],
-                        q_fallback: bool) -> Tuple[Optional[bool], Optional[torch.Tensor]]:
-    """(apply the output-channel scales?, skew as a device scalar or None).
-    A forced value wins; without one the skew decides, and without a
-    Hessian diagonal the scales apply. In fallback mode only a forced True
-    applies them. The decision is None when the skew makes it: the caller
-    then selects on the device and reads it back once, at the end."""
+                        q_fallback: bool) -> Tuple[Optional[bool], bool]:
+    """(apply the output-channel scales?, is the skew wanted?). A forced
+    value wins; without one the skew decides, and without a Hessian diagonal
+    the scales apply. In fallback mode only a forced True applies them. The
+    decision is None when the skew makes it: it is then taken on the device
+    and read back once, at the end."""
     if q_fallback:
-        return bool(forced), None
+        return bool(forced), False
     if H_diag is None:
-        return (True if forced is None else bool(forced)), None
-    return (None if forced is None else bool(forced)), _skew_tensor(H_diag)
+        return (True if forced is None else bool(forced)), False
+    return (None if forced is None else bool(forced)), True
 
 
 def _check_inputs(weight: torch.Tensor, su: torch.Tensor, sv: torch.Tensor, had_dim: int) -> None:
@@ -145,50 +149,46 @@ def regularize(weight: torch.Tensor, su: torch.Tensor, sv: torch.Tensor,
     (regularize.py:83-211). ``weight`` is not modified. ``quant_args`` may
     force ``apply_out_scales``; when given, its ``zeros`` entry is set to
     whether W had no energy at all."""
-    from ._native import block_rms_from_slices, hadamard128_scaled
+    from ._native import hadamard128_scaled, input_scales, output_scales
 
     _check_inputs(weight, su, sv, had_dim)
     k, n = weight.shape
     dev = weight.device
     forced = None if quant_args is None else quant_args.get("apply_out_scales")
-    apply_out, skew_t = _out_scale_decision(H_diag, forced, q_fallback)
+    apply_out, skew_needed = _out_scale_decision(H_diag, forced, q_fallback)
     w = weight.contiguous()
 
-    # Pass 1: output-channel scales from the column RMS, normalised by
-    # their mean unless W has no energy (the scales then stay as they are).
-    # Nothing is read back here: the decisions select on the device and
-    # come back together after the last pass.
-    out_scales = block_rms(w, dim=0, keepdim=True)
-    mean = out_scales.mean()
-    live = mean > _TINY
-    out_scales /= torch.where(live, mean, torch.ones_like(mean))
-    if forced is not None and not bool(live):
-        apply_out = True          # a forced decision on an all-zero W applies the scales
-    dead_cols = out_scales.abs() < _TINY
-    sv = sv.to(device=dev, dtype=torch.float32).reshape(1, n).clone()
-    if apply_out is None:
-        apply_t = skew_t < OUT_SCALE_SKEW_CUTOFF
-        out_scales.copy_(torch.where(dead_cols & apply_t, ZERO_FLOOR, out_scales))
-        sv = torch.where(apply_t, (sv * out_scales + EPS).float(), sv)
-    elif apply_out:
-        out_scales[dead_cols] = ZERO_FLOOR
-        sv = (sv * out_scales + EPS).float()
+    # Pass 1: output-channel scales from the column RMS, normalised by their
+    # mean unless W has no energy (the scales then stay as they are). Nothing
+    # is read back here: the decisions are taken on the device and come back
+    # together after the last pass.
+    vec = dict(dtype=torch.float32, device=dev)
+    out_scales = torch.empty((1, n), **vec)
+    divisor, sv_out = torch.empty(n, **vec), torch.empty((1, n), **vec)
+    flags = torch.zeros(3, dtype=torch.float64, device=dev)
+    sv = sv.to(device=dev, dtype=torch.float32).reshape(n).contiguous()
+    diag = None
+    if skew_needed:
+        if H_diag.dtype == torch.float32 and H_diag.device == dev and H_diag.dim() == 1 \
+                and H_diag.numel() > 0 and H_diag.stride(0) > 0:
+            diag = H_diag
+        else:
+            flags[1] = _skew_tensor(H_diag)
+    output_scales(w, sv, 2 if apply_out is None else int(apply_out), forced is not None,
+                  out_scales, divisor, sv_out, flags, diag)
 
     # Pass 2: W / sv and the right transform, with the row slice sums of
     # squares for the input-channel scales.
     work = torch.empty_like(w)
-    slice_sq = torch.empty((k, n // RMS_SLICE), dtype=torch.float32, device=dev)
-    hadamard128_scaled(w, work, 1, divisor=sv.reshape(n).contiguous(), slice_sumsq=slice_sq)
-    sv[dead_cols] = 0.0
-    in_scales = torch.empty((k, 1), dtype=torch.float32, device=dev)
-    block_rms_from_slices(slice_sq, in_scales, n)
+    slice_sq = torch.empty((k, n // RMS_SLICE), **vec)
+    hadamard128_scaled(w, work, 1, divisor=divisor, slice_sumsq=slice_sq)
+    in_scales, su_out = torch.empty((k, 1), **vec), torch.empty((k, 1), **vec)
+    su = su.to(device=dev, dtype=torch.float32).reshape(k).contiguous()
+    input_scales(slice_sq, su, in_scales, su_out, n)
     del slice_sq
-    in_scales[in_scales.abs() < _TINY] = ZERO_FLOOR
-    su = su.to(device=dev, dtype=torch.float32).reshape(k, 1)
-    su = (su * in_scales / (-CODEBOOK_SCALE) + EPS).float()
 
     # Pass 3: divide by su and the left transform, in place.
-    hadamard128_scaled(work, work, 0, divisor=su.reshape(k).contiguous())
+    hadamard128_scaled(work, work, 0, divisor=su_out)
 
     if skip_g_scale:
         g_scale = 1.0
@@ -198,19 +198,14 @@ def regularize(weight: torch.Tensor, su: torch.Tensor, sv: torch.Tensor,
         g_scale = float(g_scale_fn(work))
         if not g_scale > 0.0:
             raise ValueError(f"g_scale_fn returned a non-positive scale: {g_scale}")
-    work *= g_scale
-    su /= g_scale
-    flags = [live.to(torch.float64)]
-    if skew_t is not None:
-        flags += [skew_t.to(torch.float64), (skew_t < OUT_SCALE_SKEW_CUTOFF).to(torch.float64)]
-    flags = torch.stack(flags).tolist()          # the one read-back of the pipeline
-    zeros = not flags[0]
-    skew = flags[1] if skew_t is not None else None
-    if apply_out is None:
-        apply_out = bool(flags[2])
+        work *= g_scale
+        su_out /= g_scale
+    live, skew, applied = flags.tolist()         # the one read-back of the pipeline
+    zeros = not live
     if quant_args is not None:
         quant_args["zeros"] = zeros
-    return RegularizeResult(apply_out_scales=bool(apply_out), weight=work, g_scale=g_scale,
-                            su=su, sv=sv, out_channel_scales=out_scales,
-                            in_channel_scales=in_scales, zeros=zeros, skew_factor=skew)
+    return RegularizeResult(apply_out_scales=bool(applied), weight=work, g_scale=g_scale,
+                            su=su_out, sv=sv_out, out_channel_scales=out_scales,
+                            in_channel_scales=in_scales, zeros=zeros,
+                            skew_factor=skew if skew_needed else None)
 

@@ -62,6 +62,30 @@ int exl3_decode_weight(const uint16_t* packed, const float* su, const float* sv,
 int exl3_block_rms_from_slices(const float* slice_sumsq, float* out, int64_t outputs, int64_t n,
                                int64_t slices, void* stream);
 
+/* The input-channel step of regularize (regularize.py:171-181): scales[r] as
+ * exl3_block_rms_from_slices, 0.1 where that is below 1e-30, and su_out[r] =
+ * su[r] * scales[r] / -1.24371088 + 1e-10. */
+int exl3_input_scales(const float* slice_sumsq, const float* su, float* scales, float* su_out,
+                      int64_t rows, int64_t n, int64_t slices, void* stream);
+
+/* The output-channel step of regularize (regularize.py:102-168) for a
+ * rows x cols matrix x: scales = its column RMS (32-row slices, as
+ * exl3_block_rms) divided by their mean unless that is below 1e-30 (no
+ * energy); where the scales apply, columns whose scale is below 1e-30 get
+ * 0.1 and divisor[c] = sv[c] * scales[c] + 1e-10, elsewhere divisor = sv;
+ * sv_out = divisor with 0 for those columns. decide: 0 the scales do not
+ * apply, 1 they do, 2 they do if the skew is below 0.15; forced != 0: they
+ * also apply to a matrix without energy. With diag (diag_len values,
+ * diag_stride apart; may be NULL) the skew is the share of sum(sqrt(diag))
+ * that its largest diag_len / 50 values hold and is written to flags[1];
+ * without it flags[1] is read when decide = 2. flags (device doubles):
+ * {has energy, skew, applied}. workspace: exl3_block_rms_workspace(rows,
+ * cols, 0, 32) floats. */
+int exl3_output_scales(const float* x, int64_t rows, int64_t cols, const float* diag,
+                       int64_t diag_stride, int64_t diag_len, const float* sv, int decide,
+                       int forced, float* workspace, int64_t workspace_elems, float* scales,
+                       float* divisor, float* sv_out, double* flags, void* stream);
+
 /* Replaces block_rms (regularize.py:41-56): out = sqrt(S / n), S the sum of
  * squares along `dim` (0: over rows, one output per column; 1: over
  * columns, one per row) taken in slices of `blocksize` whose sums are

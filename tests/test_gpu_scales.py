@@ -1,0 +1,120 @@
+"""The scale kernels of regularize at the ends of their ranges: the skew by
+radix selection against a float64 sort (ties at the threshold, lengths
+around the 1/50 cut, a strided diagonal, NaN), the scale vectors against
+float64, and the row RMS at slice counts around the chunk and batch sizes."""
+
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+EPS32 = 2.0 ** -24
+
+
+def _run(torch, x, diag, decide=2, forced=False, sv=None):
+    from exl3_intel_arc_quantizer_amd._native import output_scales
+    n = x.shape[1]
+    sv = torch.ones(n, device="cuda") if sv is None else sv
+    out = [torch.empty(n, device="cuda") for _ in range(3)]
+    flags = torch.zeros(3, dtype=torch.float64, device="cuda")
+    output_scales(x, sv, decide, forced, *out, flags, diag)
+    return [t.cpu().numpy().astype(np.float64) for t in out], flags.tolist()
+
+
+@pytest.mark.parametrize("length", [1, 49, 50, 99, 100, 1023, 4097, 12288])
+def test_skew(length):
+    import torch
+    rng = np.random.default_rng(length)
+    x = torch.randn(128, 128, device="cuda")
+    for case in ("random", "ties", "strided"):
+        d = (rng.random(length) * 4.0).astype(np.float32)
+        if case == "ties":
+            d = np.round(d)
+        if case == "strided":
+            host = np.zeros((length, 3), dtype=np.float32)
+            host[:, 1] = d
+            diag = torch.from_numpy(host).cuda()[:, 1]
+        else:
+            diag = torch.from_numpy(d).cuda()
+        root = np.sort(np.sqrt(d).astype(np.float64))[::-1]
+        want = root[:length // 50].sum() / root.sum()
+        _, flags = _run(torch, x, diag)
+        # Double sums of the same float32 roots, two roundings to float32 and
+        # a division (one more each for the roots).
+        assert flags[1] == pytest.approx(want, rel=4 * EPS32, abs=0.0), case
+        assert flags[2] == float(np.float32(flags[1]) < np.float32(0.15))
+    d[0] = np.nan
+    assert math.isnan(_run(torch, x, torch.from_numpy(d).cuda())[1][1])
+
+
+@pytest.mark.parametrize("k,n", [(32, 1), (128, 63), (1056, 65), (4128, 1100)])
+def test_output_scales(k, n):
+    import torch
+    rng = np.random.default_rng(n)
+    w = rng.standard_normal((k, n)).astype(np.float32)
+    if n > 8:
+        w[:, 5] = 0.0
+    sv = (rng.random(n) + 0.5).astype(np.float32)
+    col = np.sqrt((w.astype(np.float64) ** 2).mean(axis=0))
+    v = col / col.mean()
+    dead = v < 1e-30
+    floored = np.where(dead, 0.1, v)
+    x, svd = torch.from_numpy(w).cuda(), torch.from_numpy(sv).cuda()
+    # Sums of k squares in float32, slice by slice: relative error below
+    # (32 + k / 32 + 4) roundings on the sum, half of that on its root.
+    tol = (36 + k / 32) * EPS32
+    (scales, div, out), flags = _run(torch, x, None, decide=1, sv=svd)
+    np.testing.assert_allclose(scales, floored, rtol=tol)
+    np.testing.assert_allclose(div, sv * floored + 1e-10, rtol=tol)
+    np.testing.assert_allclose(out, np.where(dead, 0.0, sv * floored + 1e-10), rtol=tol)
+    assert flags[0] == 1.0 and flags[2] == 1.0
+    (scales, div, out), flags = _run(torch, x, None, decide=0, sv=svd)
+    np.testing.assert_allclose(scales, v, rtol=tol, atol=0)
+    np.testing.assert_array_equal(div, sv.astype(np.float64))
+    np.testing.assert_array_equal(out, np.where(dead, 0.0, sv.astype(np.float64)))
+    assert flags[2] == 0.0
+    # A matrix without energy: the scales apply only where the choice is forced.
+    for forced in (False, True):
+        (scales, div, out), flags = _run(torch, torch.zeros_like(x), None, 0, forced, svd)
+        assert flags[0] == 0.0 and flags[2] == float(forced) and not out.any()
+        np.testing.assert_allclose(scales, 0.1 if forced else 0.0, rtol=EPS32)
+
+
+@pytest.mark.parametrize("rows,slices", [(1, 1), (63, 2), (64, 127), (65, 128), (130, 129),
+                                         (70, 300)])
+def test_row_reduction(rows, slices):
+    import torch
+
+    from exl3_intel_arc_quantizer_amd._native import block_rms, block_rms_from_slices, input_scales
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    sq = torch.rand(rows, slices, generator=g, device="cuda")
+    sq[rows // 2] = 0.0
+    n = 32 * slices
+    ref = np.zeros(rows, dtype=np.float32)
+    host = sq.cpu().numpy()
+    for s in range(slices):     # slice order, float32
+        ref = host[:, 0].copy() if s == 0 else ref + host[:, s]
+    ref = np.sqrt(ref / np.float32(n))
+    out = torch.empty(rows, device="cuda")
+    block_rms_from_slices(sq, out, n)
+    np.testing.assert_array_equal(out.cpu().numpy(), ref)
+    su = torch.rand(rows, generator=g, device="cuda") + 0.5
+    scales, su_out = torch.empty_like(su), torch.empty_like(su)
+    input_scales(sq, su, scales, su_out, n)
+    want = np.where(ref < 1e-30, np.float32(0.1), ref)
+    np.testing.assert_array_equal(scales.cpu().numpy(), want)
+    np.testing.assert_allclose(su_out.cpu().numpy(),
+                               su.cpu().numpy().astype(np.float64) * want / -1.24371088 + 1e-10,
+                               rtol=4 * EPS32)
+    # Both dimensions of block_rms go through the same reductions.
+    x = torch.randn(n, rows, generator=g, device="cuda")
+    for dim in (0, 1):
+        y = x if dim == 0 else x.t().contiguous()
+        block_rms(y, out, dim)
+        np.testing.assert_allclose(out.cpu().numpy(),
+                                   np.sqrt((x.cpu().numpy().astype(np.float64) ** 2).mean(0)),
+                                   rtol=(36 + slices) * EPS32)
