@@ -64,6 +64,9 @@ _SIGNATURES = {
     "exl3_block_rms_workspace": (_c_i64, [_c_i64, _c_i64, _c_int, _c_int]),
     "exl3_cholesky_diag_block": (_c_int, [_c_vp, _c_i64, _c_int, _c_i64, _c_vp, _c_vp]),
     "exl3_cholesky_block_order": (_c_int, []),
+    "exl3_cholesky": (_c_int, [_c_vp, _c_i64, _c_vp, _c_vp, _c_vp]),
+    "exl3_cholesky_inverse_elems": (_c_i64, [_c_i64]),
+    "exl3_block_fold": (_c_int, [_c_vp, _c_vp, _c_vp, _c_i64, _c_vp]),
     "exl3_ldlq_gather": (_c_int, [_c_vp, _c_int, _c_i64, _c_vp, _c_vp]),
     "exl3_ldlq_scatter": (_c_int, [_c_vp, _c_int, _c_i64, _c_vp, _c_vp, _c_vp]),
 }
@@ -666,6 +669,42 @@ def cholesky_diag_block(a, j0: int, nb: int, info) -> None:
         _check(load_library().exl3_cholesky_diag_block(a.data_ptr() + 4 * (j0 * n + j0), n, nb,
                                                        j0, info.data_ptr(), _stream(dev)),
                "cholesky_diag_block")
+
+
+def cholesky(a, info):
+    """Factor the square float32 matrix ``a`` in place (exl3_cholesky; its
+    lower triangle is read, what lies above the diagonal is left as it is
+    outside the diagonal blocks). Returns the inverses of the factor's 16 x
+    16 diagonal tiles, (ceil(n / 16), 16, 16)."""
+    torch = _torch()
+    dev = _matrix(a, "a")
+    n = a.shape[0]
+    if a.shape[1] != n or n < 1:
+        raise RuntimeError(f"a must be square, got {tuple(a.shape)}")
+    if (not isinstance(info, torch.Tensor) or info.dtype != torch.int32
+            or info.device != a.device or info.numel() < 1):
+        raise RuntimeError("info must be an int32 tensor on a's device")
+    lib = load_library()
+    with torch.cuda.device(dev):
+        inverses = torch.empty(int(lib.exl3_cholesky_inverse_elems(n)), dtype=torch.float32,
+                               device=a.device)
+        _check(lib.exl3_cholesky(a.data_ptr(), n, inverses.data_ptr(), info.data_ptr(),
+                                 _stream(dev)), "cholesky")
+    return inverses.view(-1, 16, 16)
+
+
+def block_fold(l, inverses, out) -> None:
+    """``out`` = the factor of a 16-wide block LDL from the Cholesky factor
+    ``l`` and the inverses of its diagonal tiles (exl3_block_fold)."""
+    torch = _torch()
+    dev = _matrix(l, "l")
+    n = l.shape[0]
+    _check_buffer(l, "l", torch.float32, (n, n), dev)
+    _check_buffer(out, "out", torch.float32, (n, n), dev)
+    _check_buffer(inverses, "inverses", torch.float32, (n // 16, 16, 16), dev)
+    with torch.cuda.device(dev):
+        _check(load_library().exl3_block_fold(l.data_ptr(), inverses.data_ptr(), out.data_ptr(),
+                                              n, _stream(dev)), "block_fold")
 
 
 LDLQ_BLOCK_FIELDS = ("w", "comp", "wq", "err", "states", "n", "tile0", "reserved")

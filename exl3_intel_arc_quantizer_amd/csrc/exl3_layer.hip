@@ -20,13 +20,12 @@
 //   column_scales_kernel / output_scales_kernel
 //       regularize's output-channel scales from the column slice sums, with
 //       the skew decision on the device.
-//   cholesky_diag_kernel
-//       the unblocked Cholesky factorisation of one diagonal block (order
-//       <= 128) inside a blocked factorisation whose panel updates and
-//       triangular solves are GEMM-class library calls: 256 threads each
-//       hold an 8x8 sub-block of the lower triangle in registers; column k
-//       is published through a double-buffered LDS vector, one barrier per
-//       column.
+//   cholesky_diag_kernel, cholesky_solve_kernel, cholesky_update_kernel
+//       a blocked right-looking Cholesky factorisation on the fp32 matrix
+//       cores, 128 columns a panel.
+//   block_fold_kernel
+//       the block columns of the factor times the inverses of its 16 x 16
+//       diagonal tiles (a block LDL's factor).
 //   ldlq_gather_kernel / ldlq_scatter_kernel
 //       one LDLQ step's tile formation and write-back for every 16-row block
 //       of an encoder call, one 256-thread workgroup per tile: thread p moves
@@ -504,106 +503,475 @@ __global__ void __launch_bounds__(SC_THREADS)
   }
 }
 
-// -------------------------------------------------------- Cholesky block
+// -------------------------------------------------------------- Cholesky
+//
+// Blocked right-looking factorisation in panels of 128 columns, two launches
+// a panel: the panel's rows below its diagonal block are solved against it
+// (cholesky_solve_kernel), then every 128 x 128 tile of the trailing lower
+// triangle loses X_i X_j^T (cholesky_update_kernel), whose first workgroup
+// takes the next diagonal block and goes on to factor it while the others
+// update. What bounds a 4096 matrix is the chain of its 32 panels, each the
+// update and factorisation of one diagonal block by one workgroup plus one
+// solve; the 23 GFLOP of updates run beside it on the fp32 matrix cores
+// (v_mfma_f32_16x16x4: fp32 products and sums).
+//
+// A diagonal block is factored in 16-column steps: one wave factors the
+// 16 x 16 diagonal tile in registers, four columns at a time, and inverts
+// it, the tiles below it are multiplied by that inverse, and while the
+// trailing tiles are updated the first wave already takes the next diagonal
+// tile.
+// The 16 x 16 inverses are kept: the panel solve multiplies by them, and
+// they are what a block LDL folds into the factor's columns.
+// A 128-block took 87 us with one barrier per column, 28 us here (of which
+// 16 columns take about 2 us); a panel of a 4096 matrix takes 48 us (update
+// and next diagonal block 40, solve 8) where the diagonal kernel, a library
+// triangular solve and a library GEMM took 170.
+//
+// Fragments. For v_mfma_f32_16x16x4 lane l gives A[l % 16][l / 16] and
+// B[l / 16][l % 16] and holds D[4 (l / 16) + r][l % 16] in register r. Over
+// 16 values of k, lane l's step-t value may be k = 4 (l / 16) + t, in A and
+// B alike, so a lane's four values are one 16-byte load along k.
 
-constexpr int CH_NB = 128;              // largest block order
-constexpr int CH_SB = 8;                // rows / columns of a thread's sub-block
-constexpr int CH_GRID = CH_NB / CH_SB;  // 16 x 16 sub-blocks
-constexpr int CH_THREADS = CH_GRID * CH_GRID;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// Factors the nb x nb block at `a` (row-major, leading dimension lda,
-// lower triangle read) in place: L on and below the diagonal, zeros above.
+constexpr int CH_NB = 128;               // panel width, largest block order
+constexpr int CH_T = 16;                 // tile
+constexpr int CH_TILES = CH_NB / CH_T;
+constexpr int CH_LD = CH_NB + 4;         // LDS row stride: 16-byte aligned, rows 4 banks apart
+constexpr int CH_WLD = CH_T + 4;
+constexpr int CH_THREADS = 256;
+constexpr int CH_KC = 32, CH_KLD = CH_KC + 4;  // columns staged at a time by the update
+
+// acc += A B over 16 values of k.
+__device__ __forceinline__ f32x4 mfma16(f32x4 a, f32x4 b, f32x4 acc) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t], b[t], acc, 0, 0, 0);
+  return acc;
+}
+
+// 1 / sqrt(p) to an ulp, from the hardware estimate; p below 2^-100 is scaled,
+// since the estimate takes a subnormal for zero.
+__device__ __forceinline__ float inverse_sqrt(float p) {
+  const float plain = __builtin_amdgcn_rsqf(p);
+  const float tiny = __builtin_amdgcn_rsqf(p * 0x1p64f) * 0x1p32f;
+  return p < 0x1p-100f ? tiny : plain;
+}
+
+// The value of `v` in lane `src` of the wave.
+__device__ __forceinline__ float lane_value(float v, int src) {
+  return __int_as_float(__builtin_amdgcn_ds_bpermute(4 * src, __float_as_int(v)));
+}
+__device__ __forceinline__ float uniform_value(float v, int src) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
+}
+__device__ __forceinline__ float pick(const float (&v)[4], int i) {
+  const float lo = i & 1 ? v[1] : v[0], hi = i & 1 ? v[3] : v[2];
+  return i & 2 ? hi : lo;
+}
+
+// Factors a 16 x 16 tile held in m (the whole symmetric tile in D layout:
+// m[t] = element [4 (l / 16) + t][l % 16]). Writes the factor to d (LDS, row
+// stride CH_LD, zeros above the diagonal) and its inverse to s_inv. One wave,
+// and no global store in it: each would be waited for on the way.
+//
+// Four columns at a time: rows 4 p .. 4 p + 3 of the symmetric remainder are
+// columns 4 p .. 4 p + 3, one row per lane, in lanes 16 p .. 16 p + 15; every
+// 16-lane group takes a copy and factors them (6 multiply-adds against a
+// scalar), and the remainder loses their product in one matrix instruction
+// whose two operands are the same register. The inverse advances beside it:
+// rows 4 p .. of the remainder of I are divided by the 4 x 4 diagonal part
+// in place, and the rest loses the columns times those rows. Entries of
+// finished rows and columns are garbage that no later one reads.
+__device__ __forceinline__ void factor_tile(f32x4 m, float* d, float* s_inv, int lane,
+                                            int64_t index, int32_t* info) {
+  const int r = lane & 15, g = lane >> 4;
+  f32x4 w;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) w[t] = 4 * g + t == r ? 1.0f : 0.0f;
+  int bad = 0;
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    float v[4], rs[4], x[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) v[c] = lane_value(m[c], 16 * p + r);
+    float l[4][4];  // the 4 x 4 diagonal part, uniform
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const float pivot = uniform_value(v[c], 4 * p + c);
+      if (bad == 0 && !(pivot > 0.0f)) bad = 4 * p + c + 1;
+      rs[c] = inverse_sqrt(pivot);
+      // The column times 1 / root (LAPACK's potf2 scaling); the diagonal,
+      // which no other entry waits for, is the root with one correction (its
+      // residual is exact in fp32).
+      const float scaled = v[c] * rs[c];
+#pragma unroll
+      for (int e = c + 1; e < 4; ++e) {
+        l[e][c] = uniform_value(scaled, 4 * p + e);
+        v[e] = fmaf(-l[e][c], scaled, v[e]);
+      }
+      const float root = pivot * rs[c];
+      const float fixed = fmaf(fmaf(-root, root, pivot), 0.5f * rs[c], root);
+      v[c] = r == 4 * p + c ? fixed : scaled;
+    }
+    if (g == 0) {
+      f32x4 q;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) q[c] = 4 * p + c <= r ? v[c] : 0.0f;
+      *reinterpret_cast<f32x4*>(d + r * CH_LD + 4 * p) = q;
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      float y = w[c];
+#pragma unroll
+      for (int e = 0; e < c; ++e) y = fmaf(-l[c][e], x[e], y);
+      x[c] = y * rs[c];
+    }
+    if (g == p) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        // The inverse is lower triangular: nothing above the diagonal.
+        s_inv[(4 * p + c) * CH_WLD + r] = 4 * p + c >= r ? x[c] : 0.0f;
+      }
+    }
+    if (p < 3) {
+      const float a = pick(v, g);  // column 4 p + g, row r: A and, transposed, B
+      float rows[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) rows[c] = lane_value(x[c], 16 * p + r);
+      m = __builtin_amdgcn_mfma_f32_16x16x4f32(-a, a, m, 0, 0, 0);
+      w = __builtin_amdgcn_mfma_f32_16x16x4f32(-a, pick(rows, g), w, 0, 0, 0);
+    }
+  }
+  if (bad != 0 && lane == 0) atomicCAS(info, 0, (int32_t)(index + bad));
+}
+
+// X_i X_j^T, X the 16 columns from column k0 of the block in LDS.
+__device__ __forceinline__ f32x4 tile_product(const float* s, int i, int j, int k0, int lane) {
+  const int r = lane & 15, g = lane >> 4;
+  const f32x4 a = *reinterpret_cast<const f32x4*>(s + (16 * i + r) * CH_LD + k0 + 4 * g);
+  const f32x4 b = *reinterpret_cast<const f32x4*>(s + (16 * j + r) * CH_LD + k0 + 4 * g);
+  const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  return mfma16(a, b, zero);
+}
+
+// Diagonal tile t of the block in LDS, its lower triangle mirrored.
+__device__ __forceinline__ f32x4 symmetric_tile(const float* s, int t, int lane) {
+  const int r = lane & 15, g = lane >> 4;
+  const float* d = s + 16 * t * (CH_LD + 1);
+  f32x4 m;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int row = 4 * g + q;
+    m[q] = row >= r ? d[row * CH_LD + r] : d[r * CH_LD + row];
+  }
+  return m;
+}
+
+// Factors the 128 x 128 block in LDS (its lower triangle; tiles past
+// `tiles` are left alone). inv receives the inverses of its 16 x 16 diagonal
+// tiles, back to back (may be NULL). All four waves.
+__device__ __forceinline__ void factor_block(float* s, float* s_inv, int tiles, float* __restrict__ inv,
+                             int64_t offset, int32_t* info) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  auto store_inverse = [&](int t) {
+    static_assert(CH_T * CH_T == CH_THREADS, "one element of a tile per thread");
+    if (inv)
+      inv[t * CH_THREADS + threadIdx.x] =
+          s_inv[(threadIdx.x / CH_T) * CH_WLD + threadIdx.x % CH_T];
+  };
+  if (wave == 0) factor_tile(symmetric_tile(s, 0, lane), s, s_inv, lane, offset, info);
+  __syncthreads();
+  for (int kb = 0; kb + 1 < tiles; ++kb) {
+    const int k0 = 16 * kb;
+    store_inverse(kb);
+    // X_t = S_t inverse^T for the tiles below the diagonal one.
+    const int r = lane & 15, g = lane >> 4;
+    const f32x4 w = *reinterpret_cast<const f32x4*>(s_inv + r * CH_WLD + 4 * g);
+    for (int t = kb + 1 + wave; t < tiles; t += 4) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(s + (16 * t + r) * CH_LD + k0 + 4 * g);
+      const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+      const f32x4 d = mfma16(x, w, zero);
+      // Every lane's loads above are done before any lane of the wave
+      // stores: one wave owns the tile and its instructions are in order.
+#pragma unroll
+      for (int q = 0; q < 4; ++q) s[(16 * t + 4 * g + q) * CH_LD + k0 + r] = d[q];
+    }
+    __syncthreads();
+    if (wave == 0) {
+      const f32x4 m = symmetric_tile(s, kb + 1, lane) - tile_product(s, kb + 1, kb + 1, k0, lane);
+      factor_tile(m, s + (k0 + 16) * (CH_LD + 1), s_inv, lane, offset + k0 + 16, info);
+    } else {
+      // The other trailing tiles, lower triangle, dealt over waves 1 .. 3.
+      const int left = tiles - kb - 2;  // tile rows below the next diagonal tile
+      for (int u = wave - 1; u < left * (left + 3) / 2; u += 3) {
+        // Tile row i has i + 2 tiles, tile columns kb + 1 .. kb + 2 + i.
+        int i = 0, j = u;
+        while (j > i + 1) j -= i++ + 2;
+        const int ti = kb + 2 + i, tj = kb + 1 + j;
+        const f32x4 d = tile_product(s, ti, tj, k0, lane);
+        float* c = s + (16 * ti + 4 * g) * CH_LD + 16 * tj + r;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) c[t * CH_LD] -= d[t];
+      }
+    }
+    __syncthreads();
+  }
+  store_inverse(tiles - 1);
+}
+
+// The lower triangle of the factored block to a (leading dimension lda),
+// zeros above the diagonal, the first nb rows and columns only.
+__device__ __forceinline__ void store_block(const float* s, float* __restrict__ a, int64_t lda,
+                                            int nb) {
+#pragma unroll 16
+  for (int e = 0; e < CH_NB * CH_NB / CH_THREADS; ++e) {
+    const int i = threadIdx.x + e * CH_THREADS, r = i / CH_NB, c = i % CH_NB;
+    const float v = c <= r ? s[r * CH_LD + c] : 0.0f;
+    if (r < nb && c < nb) a[r * lda + c] = v;
+  }
+}
+
+// Factors the nb x nb block at `a` (row-major, leading dimension lda, lower
+// triangle read) in place: L on and below the diagonal, zeros above.
 // Positions past nb act as an identity block and are never stored. A pivot
 // that is not positive (or NaN) sets *info to offset + k + 1 if *info is
 // still 0; the factorisation then carries on and its result is meaningless,
 // as LAPACK's potrf leaves it.
 __global__ void __launch_bounds__(CH_THREADS)
     cholesky_diag_kernel(float* __restrict__ a, int64_t lda, int nb, int64_t offset,
-                         int32_t* __restrict__ info) {
-  __shared__ float col[2][CH_NB];
-  const int t = threadIdx.x;
-  const int bi = t / CH_GRID, bj = t % CH_GRID;
-  const bool active = bj <= bi;
-  const int i0 = bi * CH_SB, j0 = bj * CH_SB;
-
-  float v[CH_SB][CH_SB];
-#pragma unroll
-  for (int r = 0; r < CH_SB; ++r) {
-#pragma unroll
-    for (int c = 0; c < CH_SB; ++c) {
-      const int i = i0 + r, j = j0 + c;
-      float x = 0.0f;
-      if (i >= nb || j >= nb)
-        x = (i == j) ? 1.0f : 0.0f;
-      else if (active && j <= i)
-        x = a[(int64_t)i * lda + j];
-      v[r][c] = x;
-    }
-  }
-  if (bj == 0) {
-#pragma unroll
-    for (int r = 0; r < CH_SB; ++r) col[0][i0 + r] = v[r][0];
+                         float* __restrict__ inv, int32_t* __restrict__ info) {
+  __shared__ __attribute__((aligned(16))) float s[CH_NB * CH_LD];
+  __shared__ __attribute__((aligned(16))) float s_inv[CH_T * CH_WLD];
+  // Loads at clamped positions, none behind a branch, so that they are in
+  // flight together.
+#pragma unroll 32
+  for (int e = 0; e < CH_NB * CH_NB / CH_THREADS; ++e) {
+    const int i = threadIdx.x + e * CH_THREADS, r = i / CH_NB, c = i % CH_NB;
+    const float v = a[(int64_t)(r < nb ? r : nb - 1) * lda + (c < nb ? c : nb - 1)];
+    s[r * CH_LD + c] = (r < nb && c <= r) ? v : (r == c ? 1.0f : 0.0f);
   }
   __syncthreads();
+  factor_block(s, s_inv, (nb + CH_T - 1) / CH_T, inv, offset, info);
+  store_block(s, a, lda, nb);
+}
 
-  // Only lower-triangle elements are ever published or stored, so the
-  // updates below run unmasked over whole sub-blocks: what they write above
-  // the diagonal (from stale column entries of rows < k) is never read.
-  bool failed = false;
-  for (int kb = 0; kb < CH_GRID; ++kb) {
+// Rows [r0, n) of panel column j0 (128 wide): X = A L11^-T against the
+// factored block L11 at (j0, j0), 16 columns at a time: X_c = (A_c -
+// sum_{k < c} X_k L_ck^T) W_c^T, W_c the inverse of L11's diagonal tile c.
+// One wave per 16 rows, its 16 x 128 strip in registers; X_c passes through
+// a wave-private LDS tile to become an operand.
+__global__ void __launch_bounds__(CH_THREADS)
+    cholesky_solve_kernel(float* __restrict__ a, int64_t n, int64_t j0,
+                          const float* __restrict__ inv) {
+  __shared__ __attribute__((aligned(16))) float s_l[CH_NB * CH_LD];
+  __shared__ __attribute__((aligned(16))) float s_x[CH_THREADS / 64][CH_T * CH_WLD];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const float* l11 = a + j0 * n + j0;
+#pragma unroll 32
+  for (int e = 0; e < CH_NB * CH_NB / CH_THREADS; ++e) {
+    const int i = threadIdx.x + e * CH_THREADS;
+    s_l[i / CH_NB * CH_LD + i % CH_NB] = l11[i / CH_NB * n + i % CH_NB];
+  }
+  const int64_t row0 = j0 + CH_NB + (int64_t)blockIdx.x * 64 + wave * 16 + 4 * g;
+  float* strip = a + row0 * n + j0 + r;
+  f32x4 acc[CH_TILES];
 #pragma unroll
-    for (int kc = 0; kc < CH_SB; ++kc) {
-      const int k = kb * CH_SB + kc;
-      const float* ck = col[kc & 1];
-      const float d = ck[k];
-      if (t == 0 && !failed && !(d > 0.0f)) {
-        failed = true;
-        atomicCAS(info, 0, (int32_t)(offset + k + 1));
-      }
-      const float s = sqrtf(d);
-      const float rs = 1.0f / s;
-      if (active && bj >= kb) {
-        float li[CH_SB], lj[CH_SB];
+  for (int c = 0; c < CH_TILES; ++c) {
 #pragma unroll
-        for (int r = 0; r < CH_SB; ++r) li[r] = ck[i0 + r] * rs;
-#pragma unroll
-        for (int c = 0; c < CH_SB; ++c) lj[c] = ck[j0 + c] * rs;
-        if (bj == kb) {
-          // Column k is final (L[k][k] = s, below it the column times 1/s,
-          // the scaling of LAPACK's potf2); columns after it are updated.
-#pragma unroll
-          for (int r = 0; r < CH_SB; ++r) v[r][kc] = li[r];
-          if (bi == kb) v[kc][kc] = s;
-#pragma unroll
-          for (int r = 0; r < CH_SB; ++r) {
-#pragma unroll
-            for (int c = kc + 1; c < CH_SB; ++c) v[r][c] = fmaf(-li[r], lj[c], v[r][c]);
-          }
-        } else {
-#pragma unroll
-          for (int r = 0; r < CH_SB; ++r) {
-#pragma unroll
-            for (int c = 0; c < CH_SB; ++c) v[r][c] = fmaf(-li[r], lj[c], v[r][c]);
-          }
-        }
-        // Publish column k + 1 for the next step.
-        const int nkb = (kc == CH_SB - 1) ? kb + 1 : kb;
-        if (bj == nkb) {
-#pragma unroll
-          for (int r = 0; r < CH_SB; ++r) col[(kc + 1) & 1][i0 + r] = v[r][(kc + 1) % CH_SB];
-        }
-      }
-      __syncthreads();
+    for (int q = 0; q < 4; ++q) {
+      // Rows past the matrix read its last row; they are never stored, and
+      // rows of a strip do not mix.
+      const int64_t past = row0 + q < n ? 0 : row0 + q - (n - 1);
+      acc[c][q] = strip[(q - past) * n + 16 * c];
     }
   }
-  // L on and below the diagonal, zeros above.
+  f32x4 w[CH_TILES];
 #pragma unroll
-  for (int r = 0; r < CH_SB; ++r) {
+  for (int c = 0; c < CH_TILES; ++c) {
 #pragma unroll
-    for (int c = 0; c < CH_SB; ++c) {
-      const int i = i0 + r, j = j0 + c;
-      if (i < nb && j < nb) a[(int64_t)i * lda + j] = (j <= i && active) ? v[r][c] : 0.0f;
+    for (int t = 0; t < 4; ++t) w[c][t] = inv[c * CH_T * CH_T + r * CH_T + 4 * g + t];
+  }
+  __syncthreads();
+  float* x = s_x[wave];
+  auto operand = [&](f32x4 d) {
+    // D layout to A layout through the wave's own tile.
+#pragma unroll
+    for (int q = 0; q < 4; ++q) x[(4 * g + q) * CH_WLD + r] = d[q];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const f32x4 v = *reinterpret_cast<const f32x4*>(x + r * CH_WLD + 4 * g);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    return v;
+  };
+#pragma unroll
+  for (int c = 0; c < CH_TILES; ++c) {
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    acc[c] = mfma16(operand(acc[c]), w[c], zero);
+    if (c + 1 < CH_TILES) {
+      const f32x4 xa = -operand(acc[c]);
+#pragma unroll
+      for (int d = c + 1; d < CH_TILES; ++d)
+        acc[d] = mfma16(
+            xa, *reinterpret_cast<const f32x4*>(s_l + (16 * d + r) * CH_LD + 16 * c + 4 * g),
+            acc[d]);
     }
+  }
+#pragma unroll
+  for (int c = 0; c < CH_TILES; ++c) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (row0 + q < n) strip[q * n + 16 * c] = acc[c][q];
+    }
+  }
+}
+
+// Tile (i, j) of the trailing lower triangle (128 x 128 tiles from row and
+// column j0 + 128): C -= X_i X_j^T, X the panel at column j0. Workgroup 0 is
+// the next diagonal block, which it factors (rows past n act as an identity
+// there).
+__global__ void __launch_bounds__(CH_THREADS)
+    cholesky_update_kernel(float* __restrict__ a, int64_t n, int64_t j0, float* __restrict__ inv,
+                           int32_t* __restrict__ info) {
+  __shared__ __attribute__((aligned(16))) float s[CH_NB * CH_LD];
+  __shared__ __attribute__((aligned(16))) float s_inv[CH_T * CH_WLD];
+  static_assert(2 * CH_NB * CH_KLD <= CH_NB * CH_LD, "both operands fit where the block goes");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  // Tile b of the triangle in row order: i (i + 1) / 2 + j.
+  const int b = blockIdx.x;
+  int ti = (int)((sqrtf(8.0f * (float)b + 1.0f) - 1.0f) * 0.5f);
+  while ((ti + 1) * (ti + 2) / 2 <= b) ++ti;
+  while (ti * (ti + 1) / 2 > b) --ti;
+  const int tj = b - ti * (ti + 1) / 2;
+  const int64_t base = j0 + CH_NB;
+  const int64_t i0 = base + (int64_t)ti * CH_NB, c0 = base + (int64_t)tj * CH_NB;
+
+  float* s_a = s;
+  float* s_b = s + CH_NB * CH_KLD;
+  const int wi = (wave >> 1) * 64, wj = (wave & 1) * 64;
+  // The wave's 64 x 64 part of C. The products are summed by themselves and
+  // subtracted once: summed onto C, 128 roundings at C's size made the
+  // factor's error six times as large. Loads are at clamped positions, none
+  // behind a branch: rows and columns past the matrix are never stored.
+  auto clamp = [&](int64_t x) { return x < n ? x : n - 1; };
+  f32x4 acc[4][4] = {}, old[4][4];
+  auto fetch_c = [&]() {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const float* c = a + clamp(i0 + wi + 16 * p + 4 * g + t) * n;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) old[p][q][t] = c[clamp(c0 + wj + 16 * q + r)];
+      }
+    }
+  };
+  // Panel columns k0 .. k0 + 31 of both row ranges, one chunk in registers
+  // ahead of the one in LDS.
+  constexpr int PER = CH_NB * CH_KC / CH_THREADS;
+  float na[PER], nb_[PER];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      const int x = threadIdx.x + e * CH_THREADS;
+      const int64_t col = j0 + k0 + x % CH_KC;
+      na[e] = a[clamp(i0 + x / CH_KC) * n + col];
+      nb_[e] = a[clamp(c0 + x / CH_KC) * n + col];
+    }
+  };
+  fetch(0);
+#pragma unroll
+  for (int k0 = 0; k0 < CH_NB; k0 += CH_KC) {
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      const int x = threadIdx.x + e * CH_THREADS;
+      s_a[x / CH_KC * CH_KLD + x % CH_KC] = na[e];
+      s_b[x / CH_KC * CH_KLD + x % CH_KC] = nb_[e];
+    }
+    __syncthreads();
+    if (k0 + CH_KC < CH_NB) {
+      fetch(k0 + CH_KC);
+    } else {
+      fetch_c();
+    }
+#pragma unroll
+    for (int kk = 0; kk < CH_KC; kk += 16) {
+      f32x4 fa[4], fb[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        fa[t] = *reinterpret_cast<const f32x4*>(s_a + (wi + 16 * t + r) * CH_KLD + kk + 4 * g);
+        fb[t] = *reinterpret_cast<const f32x4*>(s_b + (wj + 16 * t + r) * CH_KLD + kk + 4 * g);
+      }
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[p][q] = mfma16(fa[p], fb[q], acc[p][q]);
+      }
+    }
+  }
+  const bool next = b == 0;
+  if (next) __syncthreads();
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int row = wi + 16 * p + 4 * g + t, col = wj + 16 * q + r;
+        const bool in = i0 + row < n && c0 + col < n;
+        const float v = old[p][q][t] - acc[p][q][t];
+        if (next) {
+          s[row * CH_LD + col] = in && col <= row ? v : (row == col ? 1.0f : 0.0f);
+        } else if (in && c0 + col <= i0 + row) {
+          a[(i0 + row) * n + c0 + col] = v;
+        }
+      }
+    }
+  }
+  if (!next) return;
+  __syncthreads();
+  const int nb = n - base < CH_NB ? (int)(n - base) : CH_NB;
+  factor_block(s, s_inv, (nb + CH_T - 1) / CH_T, inv, base, info);
+  store_block(s, a + base * n + base, n, nb);
+}
+
+// Block column c of a block LDL factor (ldlq.py:130-142 of the reference):
+// the factor's 16 columns times the inverse of their diagonal tile, an
+// identity in the tile's own rows, zeros above. One wave per block column
+// and 64 rows; HBM-bound (the lower triangle in, the matrix out).
+__global__ void __launch_bounds__(256)
+    block_fold_kernel(const float* __restrict__ l, const float* __restrict__ inv,
+                      float* __restrict__ out, int64_t n) {
+  const int lane = threadIdx.x & 63;
+  const int r = lane & 15, g = lane >> 4;
+  const int64_t c = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (16 * c >= n) return;
+  f32x4 w;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) w[t] = inv[c * CH_T * CH_T + (4 * g + t) * CH_T + r];
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    const int64_t tile = (int64_t)blockIdx.y * 4 + p;
+    if (16 * tile >= n) return;
+    f32x4 d;
+    if (tile > c) {
+      f32x4 x;
+      const float* src = l + (16 * tile + r) * n + 16 * c + 4 * g;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) x[t] = src[t];
+      const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+      d = mfma16(x, w, zero);
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) d[t] = tile == c && r == 4 * g + t ? 1.0f : 0.0f;
+    }
+    float* dst = out + (16 * tile + 4 * g) * n + 16 * c + r;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) dst[t * n] = d[t];
   }
 }
 
@@ -861,8 +1229,43 @@ int exl3_cholesky_diag_block(float* a, int64_t lda, int nb, int64_t offset, int3
                                  (long long)lda, nb);
   if (offset < 0) return set_error("cholesky_diag_block: negative offset");
   hipLaunchKernelGGL(cholesky_diag_kernel, dim3(1), dim3(CH_THREADS), 0, as_stream(stream), a, lda,
-                     nb, offset, info);
+                     nb, offset, nullptr, info);
   return check_launch("cholesky_diag_block");
+}
+
+int exl3_cholesky(float* a, int64_t n, float* inverses, int32_t* info, void* stream) {
+  if (!a || !inverses || !info) return set_error("cholesky: NULL buffer");
+  // The tiles of a trailing triangle are counted in 32 bits.
+  if (n < 1 || n > (int64_t)CH_NB * 46000)
+    return set_error("cholesky: bad order %lld", (long long)n);
+  hipStream_t st = as_stream(stream);
+  const int first = n < CH_NB ? (int)n : CH_NB;
+  hipLaunchKernelGGL(cholesky_diag_kernel, dim3(1), dim3(CH_THREADS), 0, st, a, n, first, 0,
+                     inverses, info);
+  for (int64_t j0 = 0; j0 + CH_NB < n; j0 += CH_NB) {
+    const int64_t rows = n - j0 - CH_NB;
+    const int64_t tiles = (rows + CH_NB - 1) / CH_NB;
+    hipLaunchKernelGGL(cholesky_solve_kernel, dim3((unsigned)((rows + 63) / 64)),
+                       dim3(CH_THREADS), 0, st, a, n, j0, inverses + j0 * CH_T);
+    hipLaunchKernelGGL(cholesky_update_kernel, dim3((unsigned)(tiles * (tiles + 1) / 2)),
+                       dim3(CH_THREADS), 0, st, a, n, j0, inverses + (j0 + CH_NB) * CH_T, info);
+  }
+  return check_launch("cholesky");
+}
+
+int64_t exl3_cholesky_inverse_elems(int64_t n) {
+  return n < 1 ? -1 : (n + CH_T - 1) / CH_T * CH_T * CH_T;
+}
+
+int exl3_block_fold(const float* l, const float* inverses, float* out, int64_t n, void* stream) {
+  if (!l || !inverses || !out) return set_error("block_fold: NULL buffer");
+  if (n < CH_T || n % CH_T)
+    return set_error("block_fold: order %lld is not a positive multiple of 16", (long long)n);
+  const int64_t tiles = n / CH_T;
+  if ((tiles + 3) / 4 > 65535) return set_error("block_fold: matrix too large");
+  hipLaunchKernelGGL(block_fold_kernel, dim3((unsigned)((tiles + 3) / 4), (unsigned)((tiles + 3) / 4)),
+                     dim3(256), 0, as_stream(stream), l, inverses, out, n);
+  return check_launch("block_fold");
 }
 
 int exl3_cholesky_block_order(void) { return CH_NB; }

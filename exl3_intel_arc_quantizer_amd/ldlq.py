@@ -2,10 +2,9 @@
 (reference: exl3_quant/ldlq.py).
 
 ``block_ldl`` factors the (Hadamard-rotated, damped) Hessian H = L L^T with a
-blocked Cholesky (``cholesky_ex``: diagonal blocks factored by a HIP kernel,
-panel updates and solves as GEMM-class library calls), inverts every 16x16
-diagonal block in one batched call and folds the inverses into their block
-columns with one batched GEMM; the diagonal blocks become identities.
+blocked Cholesky in HIP kernels (``cholesky_ex``), which also leaves the
+inverses of the 16x16 diagonal blocks, and folds those into their block
+columns in one pass; the diagonal blocks become identities.
 
 ``ldlq`` quantises a (k, n) weight bottom-up: spans of ``buf_size_k`` rows
 from the last, 16-row blocks inside a span from the last. Each block's rows
@@ -57,6 +56,21 @@ class BlockLDLResult:
     block_size: int
 
 
+def _cholesky(A: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """(factor, inverses of its 16 x 16 diagonal tiles, info)."""
+    from ._native import cholesky
+    if A.dim() != 2 or A.shape[0] != A.shape[1] or A.dtype != torch.float32:
+        raise ValueError(f"cholesky_ex expects a square float32 matrix, got {A.dtype} "
+                         f"{tuple(A.shape)}")
+    if A.device.type != "cuda":
+        raise ValueError("cholesky_ex runs on the GPU; move the matrix to a cuda device")
+    info = torch.zeros(1, dtype=torch.int32, device=A.device)
+    L = torch.tril(A).contiguous()
+    if A.shape[0] == 0:
+        return L, L.new_empty((0, 16, 16)), info
+    return L, cholesky(L, info), info
+
+
 def cholesky_ex(A: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """Lower Cholesky factor of a symmetric positive-definite float32 GPU
     matrix and an int32 ``info``: 0, or the 1-based order of the first
@@ -64,32 +78,13 @@ def cholesky_ex(A: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     contract; only the lower triangle of ``A`` is read, ``A`` is not
     modified).
 
-    Left-looking and blocked by the HIP kernel's block order (128): panel j
-    gets the product of the finished columns to its left subtracted (one
-    GEMM, ``addmm_`` on the strided panel view), its diagonal block is
-    factored in LDS by ``exl3_cholesky_diag_block`` and the rows below are
-    solved against it (``solve_triangular``, a rocBLAS trsm). No host
-    synchronisation: ``info`` stays on the device."""
-    from ._native import cholesky_block_order, cholesky_diag_block
-    if A.dim() != 2 or A.shape[0] != A.shape[1] or A.dtype != torch.float32:
-        raise ValueError(f"cholesky_ex expects a square float32 matrix, got {A.dtype} "
-                         f"{tuple(A.shape)}")
-    if A.device.type != "cuda":
-        raise ValueError("cholesky_ex runs on the GPU; move the matrix to a cuda device")
-    n = A.shape[0]
-    nb = cholesky_block_order()
-    L = A.contiguous().clone()
-    info = torch.zeros(1, dtype=torch.int32, device=A.device)
-    for j0 in range(0, n, nb):
-        j1 = min(n, j0 + nb)
-        if j0 > 0:
-            L[j0:, j0:j1].addmm_(L[j0:, :j0], L[j0:j1, :j0].T, beta=1.0, alpha=-1.0)
-        cholesky_diag_block(L, j0, j1 - j0, info)
-        if j1 < n:
-            panel = L[j1:, j0:j1]
-            panel.copy_(torch.linalg.solve_triangular(L[j0:j1, j0:j1].T, panel, upper=True,
-                                                      left=False))
-    return L.tril_(), info
+    Right-looking and blocked by 128 columns on the fp32 matrix cores
+    (``exl3_cholesky``): the rows below a panel's diagonal block are solved
+    against it, then the trailing triangle is updated while one workgroup
+    already factors the next diagonal block. No host synchronisation:
+    ``info`` stays on the device."""
+    L, _, info = _cholesky(A)
+    return L, info
 
 
 def block_ldl(H: torch.Tensor, block_size: int = DEFAULT_BLOCK_SIZE,
@@ -99,8 +94,10 @@ def block_ldl(H: torch.Tensor, block_size: int = DEFAULT_BLOCK_SIZE,
     ``H`` is not modified; after a failed factorisation an internal copy is
     damped by 2 sigma_reg mean(diag) and factored again, up to
     ``max_retries`` times. The factorisation is :func:`cholesky_ex`; the
-    diagonal 16 x 16 blocks of the factor are inverted in one batched call
-    and folded into their block columns with one batched GEMM."""
+    inverses of the 16 x 16 diagonal blocks come with it and one kernel
+    folds them into their block columns (``exl3_block_fold``). Other block
+    sizes are inverted in one batched call and folded with one batched
+    GEMM."""
     if H.dim() != 2 or H.shape[0] != H.shape[1]:
         raise ValueError(f"H must be a square 2-D tensor, got shape {tuple(H.shape)}")
     if H.dtype != torch.float32:
@@ -110,18 +107,27 @@ def block_ldl(H: torch.Tensor, block_size: int = DEFAULT_BLOCK_SIZE,
     if max_retries < 0:
         raise ValueError(f"max_retries must be non-negative, got {max_retries}")
     n = H.shape[0]
-    work = H.clone()
+    work = H
     chol = None
     retries = 0
     for attempt in range(max_retries + 1):
-        chol, info = cholesky_ex(work)
+        chol, inverses, info = _cholesky(work)
         if int(info.item()) == 0:
             retries = attempt
             break
         if attempt == max_retries:
             raise torch.linalg.LinAlgError(
                 f"block_ldl: Cholesky failed after {max_retries} damping steps")
+        if work is H:
+            work = H.clone()
         work.diagonal().add_(2.0 * sigma_reg * work.diagonal().mean())
+    if block_size == 16:
+        from ._native import block_fold
+        transformed = torch.empty_like(chol)
+        block_fold(chol, inverses, transformed)
+        return BlockLDLResult(transformed=transformed, cholesky=chol, block_inverses=inverses,
+                              retries=retries, damping_applied=retries > 0, n=n,
+                              block_size=block_size)
     m = n // block_size
     # The m diagonal blocks as a strided view: [b, r, c] = chol[b bs + r, b bs + c].
     diag_view = chol.view(m, block_size, m, block_size).diagonal(dim1=0, dim2=2)

@@ -108,6 +108,25 @@ int64_t exl3_block_rms_workspace(int64_t rows, int64_t cols, int dim, int blocks
 int exl3_cholesky_diag_block(float* a, int64_t lda, int nb, int64_t offset, int32_t* info,
                              void* stream);
 
+/* Replaces torch.linalg.cholesky_ex in block_ldl (ldlq.py:76-142): factors
+ * the n x n matrix at `a` (contiguous, lower triangle read) in place into L;
+ * the entries above the diagonal outside the diagonal blocks of order 128
+ * are not touched, those inside become 0. inverses receives the inverses of
+ * L's 16 x 16 diagonal tiles, [ceil(n / 16)][16][16] (a last tile that n
+ * cuts is completed by an identity). A non-positive or NaN pivot k sets
+ * *info (device int32) to k + 1 unless it is already non-zero. Two launches
+ * per 128 columns, no host synchronisation. */
+int exl3_cholesky(float* a, int64_t n, float* inverses, int32_t* info, void* stream);
+
+/* Floats of `inverses` exl3_cholesky needs, or -1 for n < 1. */
+int64_t exl3_cholesky_inverse_elems(int64_t n);
+
+/* The fold of block_ldl (ldlq.py:120-142) for 16-wide blocks: out's block
+ * column b = l's block column b times inverses[b] below the diagonal tile,
+ * an identity in it, zeros above. n is a multiple of 16, l lower
+ * triangular; out does not overlap l. */
+int exl3_block_fold(const float* l, const float* inverses, float* out, int64_t n, void* stream);
+
 /* Largest block order exl3_cholesky_diag_block accepts (128). */
 int exl3_cholesky_block_order(void);
 
