@@ -22,6 +22,7 @@ from .build import LIB_PATH
 _LIB = None
 
 _c_int, _c_i64, _c_vp = ctypes.c_int, ctypes.c_int64, ctypes.c_void_p
+_c_float, _c_double = ctypes.c_float, ctypes.c_double
 
 # name -> (restype, argtypes)
 _SIGNATURES = {
@@ -63,6 +64,10 @@ _SIGNATURES = {
                                 _c_vp]),
     "exl3_block_rms_workspace": (_c_i64, [_c_i64, _c_i64, _c_int, _c_int]),
     "exl3_cholesky_diag_block": (_c_int, [_c_vp, _c_i64, _c_int, _c_i64, _c_vp, _c_vp]),
+    "exl3_gram": (_c_int, [_c_vp, _c_int, _c_i64, _c_i64, _c_i64, _c_float, _c_vp, _c_vp, _c_i64,
+                           _c_vp]),
+    "exl3_gram_workspace": (_c_i64, [_c_i64, _c_i64]),
+    "exl3_damp_diagonal": (_c_int, [_c_vp, _c_i64, _c_i64, _c_double, _c_float, _c_vp, _c_vp]),
     "exl3_cholesky_block_order": (_c_int, []),
     "exl3_cholesky": (_c_int, [_c_vp, _c_i64, _c_vp, _c_vp, _c_vp]),
     "exl3_cholesky_inverse_elems": (_c_i64, [_c_i64]),
@@ -645,6 +650,51 @@ def block_rms(x, out, dim: int, blocksize: int = 32) -> None:
         _check(lib.exl3_block_rms(x.data_ptr(), out.data_ptr(), rows, cols, int(dim),
                                   int(blocksize), ws.data_ptr(), ws.numel(), _stream(dev)),
                "block_rms")
+
+
+def gram_takes(x) -> bool:
+    """Whether ``gram`` takes the 2-D tensor ``x`` (exl3_gram's shape, stride
+    and alignment rules)."""
+    torch = _torch()
+    return (x.device.type == "cuda" and x.dim() == 2
+            and x.dtype in (torch.bfloat16, torch.float16) and x.shape[0] >= 1
+            and 8 <= x.shape[1] <= 1 << 20 and x.shape[1] % 8 == 0 and x.stride(1) == 1
+            and x.shape[1] <= x.stride(0) <= 1 << 24 and x.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0)
+
+
+def gram(x, scale: float):
+    """``scale * x.T @ x`` in float32 for bf16 / fp16 activations (exl3_gram)."""
+    torch = _torch()
+    if not gram_takes(x):
+        raise RuntimeError(f"gram does not take {x.dtype} {tuple(x.shape)} with strides "
+                           f"{x.stride()}")
+    tokens, d = x.shape
+    dev = x.device.index if x.device.index is not None else torch.cuda.current_device()
+    lib = load_library()
+    with torch.cuda.device(dev):
+        need = int(lib.exl3_gram_workspace(tokens, d))
+        h = torch.empty((d, d), dtype=torch.float32, device=x.device)
+        ws = torch.empty(max(need, 1), dtype=torch.float32, device=x.device)
+        _check(lib.exl3_gram(x.data_ptr(), int(x.dtype == torch.bfloat16), tokens, x.stride(0), d,
+                             float(scale), h.data_ptr(), ws.data_ptr(), ws.numel(),
+                             _stream(dev)), "gram")
+    return h
+
+
+def damp_diagonal(h, damping: float, floor: float):
+    """Damps and floors the diagonal of the square matrix ``h`` in place
+    (exl3_damp_diagonal); returns its mean before, as a device scalar."""
+    torch = _torch()
+    dev = _matrix(h, "h")
+    d = h.shape[0]
+    if h.shape[1] != d:
+        raise RuntimeError(f"h must be square, got {tuple(h.shape)}")
+    with torch.cuda.device(dev):
+        mean = torch.empty((), dtype=torch.float32, device=h.device)
+        _check(load_library().exl3_damp_diagonal(h.data_ptr(), d, d, float(damping), float(floor),
+                                                 mean.data_ptr(), _stream(dev)), "damp_diagonal")
+    return mean
 
 
 def cholesky_block_order() -> int:

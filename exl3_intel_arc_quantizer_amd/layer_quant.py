@@ -25,6 +25,7 @@ from typing import Dict, List, Optional, Tuple
 
 import torch
 
+from ._native import damp_diagonal, gram, gram_takes
 from .hadamard import HAD_DIM, blockwise_preapply_had_l_, blockwise_preapply_had_r_, \
     weight_from_quantized
 from .ldlq import (DEFAULT_BLOCK_SIZE, DEFAULT_BUF_SIZE_K, BlockLDLResult, LDLQResult,
@@ -48,24 +49,40 @@ def hessian_from_activations(x: torch.Tensor, damping_lambda: float = DEFAULT_DA
     damped by lambda * mean(diag) and floored at ``zero_floor``
     (calibration.py:359-385). Returns (H, applied damping).
 
-    bf16 / fp16 activations on the GPU go straight into a half-precision
-    GEMM with float32 output (``torch.mm(..., out_dtype=float32)``, MFMA
-    with fp32 accumulation): their products are exact in float32, so the
-    result is the float32 GEMM of the converted values up to summation
-    order, without the conversion pass and at the half-precision MFMA
-    rate."""
+    bf16 / fp16 activations on the GPU go straight onto the matrix cores
+    (``exl3_gram``): their products are exact in float32, so the result is
+    the float32 product of the converted values up to summation order, of
+    which only the lower triangle is computed. Layouts that kernel does not
+    take (an odd width, strided columns) go through a half-precision GEMM
+    with float32 output, float32 activations through a float32 GEMM. On the
+    GPU the damping and the floor are one launch, and the mean that the
+    damping is computed from is the only value read back."""
     d = x.shape[-1]
     flat = x.reshape(-1, d)
-    H = torch.zeros((d, d), dtype=torch.float32, device=x.device)
+    tokens = flat.shape[0]
+    starts = range(0, tokens, chunk_tokens)
     half = flat.device.type == "cuda" and flat.dtype in (torch.bfloat16, torch.float16)
-    for s in range(0, flat.shape[0], chunk_tokens):
-        if half:
+    # The kernels record no gradient.
+    native = flat.device.type == "cuda" and not (torch.is_grad_enabled() and x.requires_grad)
+    if native and half and len(starts) > 0 and gram_takes(flat):
+        H = gram(flat, 1.0 / tokens)
+    else:
+        H = None
+        for s in starts:
             xc = flat[s:s + chunk_tokens]
-            H += torch.mm(xc.T, xc, out_dtype=torch.float32)
-        else:
-            xf = flat[s:s + chunk_tokens].to(torch.float32)
-            H += xf.T @ xf
-    H /= max(1, flat.shape[0])
+            if half:
+                part = torch.mm(xc.T, xc, out_dtype=torch.float32)
+            else:
+                xf = xc.to(torch.float32)
+                part = xf.T @ xf
+            H = part if H is None else H.add_(part)
+        if H is None:
+            H = torch.zeros((d, d), dtype=torch.float32, device=x.device)
+        H /= max(1, tokens)
+    if native and d > 0:
+        H = H.contiguous()
+        mean = damp_diagonal(H, damping_lambda, zero_floor)
+        return H, max(1e-8, damping_lambda * mean.item())
     diag = H.diagonal()
     damp = max(1e-8, damping_lambda * diag.mean().item())
     diag.add_(damp)

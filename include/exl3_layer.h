@@ -86,6 +86,26 @@ int exl3_output_scales(const float* x, int64_t rows, int64_t cols, const float* 
                        int forced, float* workspace, int64_t workspace_elems, float* scales,
                        float* divisor, float* sv_out, double* flags, void* stream);
 
+/* The sum of hessian_from_activations (calibration.py:337-357): h = scale *
+ * X^T X for X of `tokens` rows (row stride ldx elements) and d columns, bf16
+ * (bf16 != 0) or fp16, products and sums in float32, h float32 d x d
+ * contiguous and exactly symmetric. d and ldx are multiples of 8, x is
+ * 16-byte aligned. workspace: exl3_gram_workspace floats (0 where the tokens
+ * are not shared out). */
+int exl3_gram(const uint16_t* x, int bf16, int64_t tokens, int64_t ldx, int64_t d, float scale,
+              float* h, float* workspace, int64_t workspace_elems, void* stream);
+
+/* Floats of workspace exl3_gram needs on the current device, or -1 for a
+ * shape it does not take. */
+int64_t exl3_gram_workspace(int64_t tokens, int64_t d);
+
+/* The damping of hessian_from_activations (calibration.py:359-385) on the
+ * diagonal of h (row stride ld): adds max(1e-8, lambda * mean(diagonal)),
+ * then replaces values below floor_value in magnitude by it. mean (device)
+ * receives the mean. */
+int exl3_damp_diagonal(float* h, int64_t d, int64_t ld, double lambda, float floor_value,
+                       float* mean, void* stream);
+
 /* Replaces block_rms (regularize.py:41-56): out = sqrt(S / n), S the sum of
  * squares along `dim` (0: over rows, one output per column; 1: over
  * columns, one per row) taken in slices of `blocksize` whose sums are
