@@ -55,11 +55,42 @@ hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 constexpr int HAD_N = 128;
 constexpr int HAD_RIGHT_WAVES = 4;
 
+__device__ __forceinline__ float flip(float v, uint32_t sign) {
+  return __uint_as_float(__float_as_uint(v) ^ sign);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+
 // Butterfly of lane distance h: the lane without bit h holds the lower
 // element a of each pair (a, b) and keeps a + b, its partner keeps a - b.
+// Partners are reached without the LDS crossbar: DPP quad_perm (1, 2), quad
+// reversal then row_half_mirror (4: i ^ 3 ^ 7), row_ror:8 (8), and
+// v_permlane16_swap / v_permlane32_swap (16, 32), which leave the lower
+// element of every pair in one register and the upper in the other. Through
+// ds_bpermute the 12 exchanges a row takes were the transform kernels' LDS
+// traffic (decoding a 4096 x 4096 projection took 38 us, 28 so). h must fold
+// to a constant; every lane of the wave must be active.
 __device__ __forceinline__ float had_level(float v, int lane, int h) {
-  const float p = __shfl_xor(v, h, 64);
-  return (lane & h) ? p - v : v + p;
+  const uint32_t sign = (lane & h) ? 0x80000000u : 0u;
+  switch (h) {
+    case 1: return dpp<0xB1>(v) + flip(v, sign);
+    case 2: return dpp<0x4E>(v) + flip(v, sign);
+    case 4: return dpp<0x141>(dpp<0x1B>(v)) + flip(v, sign);
+    case 8: return dpp<0x128>(v) + flip(v, sign);
+    case 16: {
+      const uint32_t u = __float_as_uint(v);
+      const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+      return __uint_as_float(r[0]) + flip(__uint_as_float(r[1]), sign);
+    }
+    default: {
+      const uint32_t u = __float_as_uint(v);
+      const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+      return __uint_as_float(r[0]) + flip(__uint_as_float(r[1]), sign);
+    }
+  }
 }
 
 // DIV: every element of column c is divided by div[c] before the transform
@@ -150,7 +181,7 @@ __global__ void __launch_bounds__(256)
 // rows g, g + 32, g + 64, g + 96 (distances 32 and 64), two columns per
 // lane, scales them and transforms the four rows across the wave. 64 KiB of
 // LDS, two workgroups per CU. A 4096 x 4096 projection at K = 4 (75 MB)
-// decodes in 38 us; unpacking, a table lookup, the un-permutation, two
+// decodes in 28 us; unpacking, a table lookup, the un-permutation, two
 // transforms and two scalings took 390 us.
 constexpr int UN_THREADS = 512;
 
@@ -172,7 +203,10 @@ __global__ void __launch_bounds__(UN_THREADS, 4)
     uint32_t* s_words = reinterpret_cast<uint32_t*>(s);
     const uint32_t* src =
         packed + ((row0 / 16 + wave) * (cols / 16) + col0 / 16) * (int64_t)(8 * K);
-    for (int j = 0; j < K; ++j) s_words[(wave * K + j) * 64 + lane] = src[j * 64 + lane];
+    // Word j sits at j ^ (j / 64 % 8): the lanes of a read are K words apart,
+    // so that those in one bank are whole 64-word blocks apart.
+    auto at = [](int j) { return j ^ ((j >> 6) & 7); };
+    for (int j = 0; j < K; ++j) s_words[at((wave * K + j) * 64 + lane)] = src[j * 64 + lane];
     __syncthreads();
     // Column 8 half + lane % 8 of tile column lane / 8. Row 2 q + (e & 1) +
     // 8 (e >> 1) of tile column cc + 8 half is encoded element i = 32 cc +
@@ -190,8 +224,8 @@ __global__ void __launch_bounds__(UN_THREADS, 4)
         for (int e = 0; e < 4; ++e) {
           const int last = (8 * q + 4 * half + e + 1) * K - 1;  // the window's last bit
           const int word = cc * K + (last >> 5);
-          const uint32_t lo = s_words[tile + word];
-          const uint32_t hi = s_words[tile + (word > 0 ? word - 1 : 8 * K - 1)];
+          const uint32_t lo = s_words[at(tile + word)];
+          const uint32_t hi = s_words[at(tile + (word > 0 ? word - 1 : 8 * K - 1))];
           const uint32_t state = __builtin_amdgcn_alignbit(hi, lo, 31 - (last & 31)) & 0xFFFFu;
           v[16 * t + 2 * q + (e & 1) + 8 * (e >> 1)] = (float)decode_state(CB, state);
         }
