@@ -134,6 +134,11 @@ def weight_from_quantized(w_hat: torch.Tensor, su: torch.Tensor,
     from ._native import unrotate
     work = w_hat if (w_hat.dtype == torch.float32 and w_hat.is_contiguous()) else \
         w_hat.to(torch.float32).contiguous()
+    su, sv = scale_vectors(su, sv, k, n, work.device)
     out = torch.empty_like(work)
-    unrotate(work, *scale_vectors(su, sv, k, n, work.device), out)
+    if torch.is_grad_enabled() and sv.requires_grad:
+        # The last step is then torch's, which records sv's gradient; x 1 is exact.
+        unrotate(work, su, torch.ones_like(sv), out)
+        return out * sv
+    unrotate(work, su, sv, out)
     return out

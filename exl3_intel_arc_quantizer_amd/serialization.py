@@ -97,6 +97,10 @@ def decode_weight_from_storage(trellis: torch.Tensor, suh: torch.Tensor, svh: to
         packed = packed.clone()
     su, sv = scale_vectors(suh, svh, k, n, packed.device)
     w = torch.empty((k, n), dtype=torch.float32, device=packed.device)
+    if torch.is_grad_enabled() and sv.requires_grad:
+        # The last step is then torch's, which records svh's gradient; x 1 is exact.
+        decode_weight(packed, su, torch.ones_like(sv), w, K, cb)
+        return (w * sv).to(trellis.device)
     decode_weight(packed, su, sv, w, K, cb)
     return w.to(trellis.device)
 

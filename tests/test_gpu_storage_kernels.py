@@ -74,3 +74,30 @@ def test_pack_alignments(K):
         extension().pack_trellis(aligned, out, K)
         extension().pack_trellis(shifted, ref, K)
         assert torch.equal(out, ref)
+
+
+def test_gradient_of_output_scales():
+    """A recorded sv gives the same weight and its gradient, the column sums
+    of the weight before the last scaling."""
+    import torch
+
+    from exl3_intel_arc_quantizer_amd.hadamard import weight_from_quantized
+    from exl3_intel_arc_quantizer_amd.serialization import (decode_weight_from_storage,
+                                                            pack_module_trellis)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    su = torch.rand(128, generator=g, device="cuda") + 0.5
+    sv = torch.rand(256, generator=g, device="cuda") + 0.5
+    w = torch.randn(128, 256, generator=g, device="cuda")
+    states = torch.randint(-32768, 32768, (8, 16, 256), generator=g, device="cuda",
+                           dtype=torch.int32).to(torch.int16)
+    trellis = pack_module_trellis(states, 4)
+    for decode in (lambda v: weight_from_quantized(w, su, v),
+                   lambda v: decode_weight_from_storage(trellis, su, v, 4)):
+        plain = decode(sv)
+        leaf = sv.clone().requires_grad_()
+        out = decode(leaf)
+        assert torch.equal(out, plain) and not plain.requires_grad
+        out.sum().backward()
+        # Sums of 128 float32 terms.
+        want, size = (plain.double() / sv).sum(dim=0), (plain.double() / sv).abs().sum(dim=0)
+        assert bool(((leaf.grad - want).abs() <= 140 * 2.0 ** -24 * size).all())
