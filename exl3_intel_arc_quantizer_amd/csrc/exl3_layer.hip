@@ -556,9 +556,9 @@ __global__ void __launch_bounds__(SC_THREADS)
 // tile.
 // The 16 x 16 inverses are kept: the panel solve multiplies by them, and
 // they are what a block LDL folds into the factor's columns.
-// A 128-block took 87 us with one barrier per column, 28 us here (of which
-// 16 columns take about 2 us); a panel of a 4096 matrix takes 48 us (update
-// and next diagonal block 40, solve 8) where the diagonal kernel, a library
+// A 128-block took 87 us with one barrier per column, 26 us here (of which
+// 16 columns take about 2 us); a panel of a 4096 matrix takes 41 us (update
+// and next diagonal block 34, solve 7.5) where the diagonal kernel, a library
 // triangular solve and a library GEMM took 170.
 //
 // Fragments. For v_mfma_f32_16x16x4 lane l gives A[l % 16][l / 16] and
@@ -598,8 +598,10 @@ __device__ __forceinline__ float lane_value(float v, int src) {
 __device__ __forceinline__ float uniform_value(float v, int src) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
 }
-__device__ __forceinline__ float pick(const float (&v)[4], int i) {
-  const float lo = i & 1 ? v[1] : v[0], hi = i & 1 ? v[3] : v[2];
+// v[i] of four registers. By value: a choice between array elements becomes a
+// choice between addresses, and the array then lives in scratch memory or LDS.
+__device__ __forceinline__ float pick(float v0, float v1, float v2, float v3, int i) {
+  const float lo = i & 1 ? v1 : v0, hi = i & 1 ? v3 : v2;
   return i & 2 ? hi : lo;
 }
 
@@ -668,12 +670,13 @@ __device__ __forceinline__ void factor_tile(f32x4 m, float* d, float* s_inv, int
       }
     }
     if (p < 3) {
-      const float a = pick(v, g);  // column 4 p + g, row r: A and, transposed, B
+      const float a = pick(v[0], v[1], v[2], v[3], g);  // column 4 p + g, row r: A and, transposed, B
       float rows[4];
 #pragma unroll
       for (int c = 0; c < 4; ++c) rows[c] = lane_value(x[c], 16 * p + r);
       m = __builtin_amdgcn_mfma_f32_16x16x4f32(-a, a, m, 0, 0, 0);
-      w = __builtin_amdgcn_mfma_f32_16x16x4f32(-a, pick(rows, g), w, 0, 0, 0);
+      const float b = pick(rows[0], rows[1], rows[2], rows[3], g);
+      w = __builtin_amdgcn_mfma_f32_16x16x4f32(-a, b, w, 0, 0, 0);
     }
   }
   if (bad != 0 && lane == 0) atomicCAS(info, 0, (int32_t)(index + bad));
@@ -862,6 +865,64 @@ __global__ void __launch_bounds__(CH_THREADS)
   }
 }
 
+// Workgroup 0's share of a trailing update: the next diagonal block (order
+// nb at `a`, leading dimension lda) loses X X^T, X its rows of the finished
+// panel at x, and is factored. This is the chain that a factorisation waits
+// for, so it is not the general tile below: X is one operand, staged once
+// and whole, only the 36 tiles on and below the diagonal are computed, nine a
+// wave (tile rows w and 7 - w), and its waves go first on their CU. Through
+// the general tile the launch took 40 us, 34 so.
+__device__ __forceinline__ void factor_next(float* s, float* s_inv, const float* __restrict__ x,
+                                            float* __restrict__ a, int64_t lda, int nb,
+                                            float* __restrict__ inv, int64_t offset,
+                                            int32_t* info) {
+  __builtin_amdgcn_s_setprio(3);
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int r = lane & 15, g = lane >> 4;
+  auto clamp = [&](int i) { return i < nb ? i : nb - 1; };
+#pragma unroll 32
+  for (int e = 0; e < CH_NB * CH_NB / CH_THREADS; ++e) {
+    const int i = threadIdx.x + e * CH_THREADS;
+    s[i / CH_NB * CH_LD + i % CH_NB] = x[clamp(i / CH_NB) * lda + i % CH_NB];
+  }
+  constexpr int OWN = CH_TILES + 1;
+  auto tile_row = [&](int u) { return u <= w ? w : CH_TILES - 1 - w; };
+  auto tile_col = [&](int u) { return u <= w ? u : u - w - 1; };
+  f32x4 acc[OWN] = {}, old[OWN];
+#pragma unroll
+  for (int u = 0; u < OWN; ++u) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      old[u][t] = a[clamp(16 * tile_row(u) + 4 * g + t) * lda + clamp(16 * tile_col(u) + r)];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < CH_NB; k += 16) {
+    auto fragment = [&](int tile) {
+      return *reinterpret_cast<const f32x4*>(s + (16 * tile + r) * CH_LD + k + 4 * g);
+    };
+    const f32x4 lo = fragment(w), hi = fragment(CH_TILES - 1 - w);
+#pragma unroll
+    for (int u = 0; u < OWN; ++u)
+      acc[u] = mfma16(u <= w ? lo : hi, fragment(tile_col(u)), acc[u]);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < OWN; ++u) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int row = 16 * tile_row(u) + 4 * g + t, col = 16 * tile_col(u) + r;
+      // Above the diagonal nothing is read.
+      s[row * CH_LD + col] =
+          row < nb && col < nb ? old[u][t] - acc[u][t] : (row == col ? 1.0f : 0.0f);
+    }
+  }
+  __syncthreads();
+  factor_block(s, s_inv, (nb + CH_T - 1) / CH_T, inv, offset, info);
+  store_block(s, a, lda, nb);
+}
+
 // Tile (i, j) of the trailing lower triangle (128 x 128 tiles from row and
 // column j0 + 128): C -= X_i X_j^T, X the panel at column j0. Workgroup 0 is
 // the next diagonal block, which it factors (rows past n act as an identity
@@ -876,11 +937,16 @@ __global__ void __launch_bounds__(CH_THREADS)
   const int r = lane & 15, g = lane >> 4;
   // Tile b of the triangle in row order: i (i + 1) / 2 + j.
   const int b = blockIdx.x;
+  const int64_t base = j0 + CH_NB;
+  if (b == 0) {
+    factor_next(s, s_inv, a + base * n + j0, a + base * n + base, n,
+                n - base < CH_NB ? (int)(n - base) : CH_NB, inv, base, info);
+    return;
+  }
   int ti = (int)((sqrtf(8.0f * (float)b + 1.0f) - 1.0f) * 0.5f);
   while ((ti + 1) * (ti + 2) / 2 <= b) ++ti;
   while (ti * (ti + 1) / 2 > b) --ti;
   const int tj = b - ti * (ti + 1) / 2;
-  const int64_t base = j0 + CH_NB;
   const int64_t i0 = base + (int64_t)ti * CH_NB, c0 = base + (int64_t)tj * CH_NB;
 
   float* s_a = s;
@@ -947,30 +1013,17 @@ __global__ void __launch_bounds__(CH_THREADS)
       }
     }
   }
-  const bool next = b == 0;
-  if (next) __syncthreads();
 #pragma unroll
   for (int p = 0; p < 4; ++p) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        const int row = wi + 16 * p + 4 * g + t, col = wj + 16 * q + r;
-        const bool in = i0 + row < n && c0 + col < n;
-        const float v = old[p][q][t] - acc[p][q][t];
-        if (next) {
-          s[row * CH_LD + col] = in && col <= row ? v : (row == col ? 1.0f : 0.0f);
-        } else if (in && c0 + col <= i0 + row) {
-          a[(i0 + row) * n + c0 + col] = v;
-        }
+        const int64_t row = i0 + wi + 16 * p + 4 * g + t, col = c0 + wj + 16 * q + r;
+        if (row < n && col <= row) a[row * n + col] = old[p][q][t] - acc[p][q][t];
       }
     }
   }
-  if (!next) return;
-  __syncthreads();
-  const int nb = n - base < CH_NB ? (int)(n - base) : CH_NB;
-  factor_block(s, s_inv, (nb + CH_T - 1) / CH_T, inv, base, info);
-  store_block(s, a + base * n + base, n, nb);
 }
 
 // Block column c of a block LDL factor (ldlq.py:130-142 of the reference):
