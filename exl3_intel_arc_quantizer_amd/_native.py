@@ -53,6 +53,8 @@ _SIGNATURES = {
     "exl3_hadamard128": (_c_int, [_c_vp, _c_vp, _c_i64, _c_i64, _c_int, _c_vp]),
     "exl3_hadamard128_scaled": (_c_int, [_c_vp, _c_vp, _c_i64, _c_i64, _c_int, _c_vp, _c_vp,
                                          _c_vp]),
+    "exl3_row_energy": (_c_int, [_c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_vp]),
+    "exl3_rotate": (_c_int, [_c_vp, _c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_vp]),
     "exl3_unrotate": (_c_int, [_c_vp, _c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_vp]),
     "exl3_decode_weight": (_c_int, [_c_vp, _c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_int, _c_int,
                                     _c_vp]),
@@ -540,6 +542,33 @@ def _scale_vector(t, name: str, numel: int, like) -> None:
             or t.device != like.device or t.numel() != numel):
         raise RuntimeError(f"{name} must be a contiguous float32 tensor of {numel} elements on "
                            f"{like.device}")
+
+
+def row_energy(x, sv, sums) -> None:
+    """Sums of squares of the 128-element segments of the rows of ``(x / sv)
+    H``, (rows, cols / 128) (exl3_row_energy)."""
+    torch = _torch()
+    dev = _matrix(x, "x")
+    rows, cols = x.shape
+    _scale_vector(sv, "sv", cols, x)
+    _check_buffer(sums, "sums", torch.float32, (rows, cols // 128), dev)
+    with torch.cuda.device(dev):
+        _check(load_library().exl3_row_energy(x.data_ptr(), sv.data_ptr(), sums.data_ptr(), rows,
+                                              cols, _stream(dev)), "row_energy")
+
+
+def rotate(x, sv, su, out) -> None:
+    """``out = H (((x / sv) H) / su)`` with blockwise order-128 transforms
+    (exl3_rotate); ``out`` must not be ``x``."""
+    torch = _torch()
+    dev = _matrix(x, "x")
+    _check_buffer(out, "out", x.dtype, tuple(x.shape), dev)
+    rows, cols = x.shape
+    _scale_vector(sv, "sv", cols, x)
+    _scale_vector(su, "su", rows, x)
+    with torch.cuda.device(dev):
+        _check(load_library().exl3_rotate(x.data_ptr(), sv.data_ptr(), su.data_ptr(),
+                                          out.data_ptr(), rows, cols, _stream(dev)), "rotate")
 
 
 def unrotate(x, su, sv, out) -> None:

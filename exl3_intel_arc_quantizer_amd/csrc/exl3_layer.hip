@@ -13,13 +13,16 @@
 //   unrotate_kernel
 //       the way back from the encoder's basis (both transforms and both
 //       scales) in one pass, from a matrix or straight from packed tiles.
+//   row_energy_kernel / rotate_kernel
+//       the way there (regularize): row energies, then both divisions and
+//       both transforms in one pass.
 //   block_rms_slices_kernel / block_rms_reduce_{columns,rows}_kernel
 //       sqrt(sum of squares / n) along one dimension: one thread per slice
 //       of `blocksize` sums its squares in order, then one thread per output
 //       accumulates the slice sums in slice order.
-//   column_scales_kernel / output_scales_kernel
-//       regularize's output-channel scales from the column slice sums, with
-//       the skew decision on the device.
+//   column_slices_kernel / output_scales_kernel
+//       regularize's column slice sums, and the output-channel scales from
+//       the column RMS, with the skew decision on the device.
 //   cholesky_diag_kernel, cholesky_solve_kernel, cholesky_update_kernel
 //       a blocked right-looking Cholesky factorisation on the fp32 matrix
 //       cores, 128 columns a panel.
@@ -292,6 +295,139 @@ __global__ void __launch_bounds__(UN_THREADS, 4)
   }
 }
 
+// Row energies of (in / sv) H_r without the transform: it is orthonormal, so
+// a 128-element segment keeps its sum of squares (and in float32 this one has
+// the fewer roundings). One read of the matrix and 1/128 of it written. A wave
+// takes two rows of a segment at a time, 16 bytes a lane, EN_LOADS of them
+// issued together. In a segment with two infinities the transform would meet
+// inf - inf, and its energy is NaN.
+constexpr int EN_LOADS = 8, EN_WAVES = 4, EN_ROWS = 2 * EN_LOADS * EN_WAVES;
+
+// Sum over the lane's half of the wave.
+__device__ __forceinline__ float half_wave_sum(float q) {
+  q = q + dpp<0xB1>(q);
+  q = q + dpp<0x4E>(q);
+  q = q + dpp<0x141>(dpp<0x1B>(q));
+  q = q + dpp<0x128>(q);
+  const uint32_t u = __float_as_uint(q);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+__global__ void __launch_bounds__(64 * EN_WAVES)
+    row_energy_kernel(const float* __restrict__ in, int64_t cols, const float* __restrict__ sv,
+                      float* __restrict__ sums) {
+  const int lane = threadIdx.x & 63, half = lane >> 5;
+  // Workgroups along the columns first.
+  const uint32_t segments = (uint32_t)(cols / HAD_N), seg = blockIdx.x % segments;
+  const int64_t row0 = (int64_t)(blockIdx.x / segments) * EN_ROWS +
+                       (int64_t)(threadIdx.x >> 6) * (2 * EN_LOADS) + half;
+  const float* src = in + row0 * cols + (int64_t)seg * HAD_N;
+  float4 x[EN_LOADS];
+#pragma unroll
+  for (int j = 0; j < EN_LOADS; ++j)
+    x[j] = reinterpret_cast<const float4*>(src + 2 * j * cols)[lane & 31];
+  const float4 d = reinterpret_cast<const float4*>(sv + (int64_t)seg * HAD_N)[lane & 31];
+#pragma unroll
+  for (int j = 0; j < EN_LOADS; ++j) {
+    const float v[4] = {x[j].x / d.x, x[j].y / d.y, x[j].z / d.z, x[j].w / d.w};
+    const float q =
+        half_wave_sum((v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]));
+    int infinities = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint64_t all = __ballot(__builtin_isinf(v[e]));
+      infinities += __popc((uint32_t)(half ? all >> 32 : all));
+    }
+    if ((lane & 31) == 0)
+      sums[(row0 + 2 * j) * segments + seg] = infinities > 1 ? __builtin_nanf("") : q;
+  }
+}
+
+// H_l (((in / sv) H_r) / su) of one 128 x 128 block per workgroup: both
+// transforms and both divisions of regularize in one read and one write,
+// once the row scales are known. The fp32 operations and their order are
+// those of the separate passes: results are bit-identical to them.
+//
+// The mirror image of unrotate_kernel. First half: each wave takes rows 4 g
+// .. 4 g + 3 for four g, two columns per lane, all its loads issued together;
+// the right transform runs across the wave, the left one starts with row
+// distances 1 and 2. Second half: wave w takes rows w / 2, w / 2 + 4, .. of
+// 64 columns, one column per lane (distances 4 .. 64). 64 KiB of LDS, two
+// workgroups per CU. A 4096 matrix (134 MB) takes 33 us, about half of it the
+// cross-lane butterflies' and the divisions' instructions, and 15 us in
+// row_energy_kernel; storing the right transform and reading it again for the
+// left one took 61.
+constexpr int RO_THREADS = 512, RO_WAVES = RO_THREADS / 64, RO_GROUPS = HAD_N / 4 / RO_WAVES;
+
+__global__ void __launch_bounds__(RO_THREADS, 4)
+    rotate_kernel(const float* __restrict__ in, const float* __restrict__ sv,
+                  const float* __restrict__ su, float* __restrict__ out, int64_t cols) {
+  __shared__ __attribute__((aligned(16))) float s[HAD_N * HAD_N];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int64_t row0 = (int64_t)blockIdx.y * HAD_N, col0 = (int64_t)blockIdx.x * HAD_N;
+
+  float2 x[RO_GROUPS][4];
+#pragma unroll
+  for (int g = 0; g < RO_GROUPS; ++g) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      x[g][j] = reinterpret_cast<const float2*>(
+          in + (row0 + 4 * (wave + RO_WAVES * g) + j) * cols + col0)[lane];
+  }
+  const float2 d = reinterpret_cast<const float2*>(sv + col0)[lane];
+#pragma unroll
+  for (int g = 0; g < RO_GROUPS; ++g) {
+    const int r0 = 4 * (wave + RO_WAVES * g);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float a = x[g][j].x / d.x, b = x[g][j].y / d.y;
+      float lo = a + b, hi = a - b;
+#pragma unroll
+      for (int h = 1; h < 64; h <<= 1) {
+        lo = had_level(lo, lane, h);
+        hi = had_level(hi, lane, h);
+      }
+      const float u = su[row0 + r0 + j];
+      x[g][j] = make_float2((lo * kHadScale) / u, (hi * kHadScale) / u);
+    }
+#pragma unroll
+    for (int h = 1; h < 4; h <<= 1) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (!(j & h)) {
+          const float2 a = x[g][j], b = x[g][j + h];
+          x[g][j] = make_float2(a.x + b.x, a.y + b.y);
+          x[g][j + h] = make_float2(a.x - b.x, a.y - b.y);
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) reinterpret_cast<float2*>(s + (r0 + j) * HAD_N)[lane] = x[g][j];
+  }
+  __syncthreads();
+
+  const int q = wave >> 1, c = (wave & 1) * 64 + lane;
+  float v[32];
+#pragma unroll
+  for (int r = 0; r < 32; ++r) v[r] = s[(q + 4 * r) * HAD_N + c];
+#pragma unroll
+  for (int h = 1; h < 32; h <<= 1) {
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      if (!(i & h)) {
+        const float a = v[i], b = v[i + h];
+        v[i] = a + b;
+        v[i + h] = a - b;
+      }
+    }
+  }
+  float* dst = out + (row0 + q) * cols + col0 + c;
+#pragma unroll
+  for (int r = 0; r < 32; ++r) dst[4 * r * cols] = v[r] * kHadScale;
+}
+
 // --------------------------------------------------------------- block RMS
 
 // Output o reduces x[o * so + t * st] over t < n, in ns slices of bs.
@@ -478,26 +614,47 @@ __device__ float diagonal_skew(const float* __restrict__ diag, int64_t stride, i
   return (float)top / (float)all;
 }
 
-// Column RMS from the slice sums, and (one more workgroup, beside them) the
-// skew of the Hessian diagonal into flags[1].
+// First pass of the column RMS (block_rms_slices_kernel's sums for dim = 0 and
+// 32-row slices), and in workgroup 0 the skew of the Hessian diagonal into
+// flags[1]: its four histogram passes over a few thousand values take 10 us
+// and wait for nothing here, so they run under the matrix's read (67 MB: 15
+// us) and not after it.
+constexpr int COL_SLICE = 32;
+
 __global__ void __launch_bounds__(SC_THREADS)
-    column_scales_kernel(const float* __restrict__ ws, float* __restrict__ scales, int64_t cols,
+    column_slices_kernel(const float* __restrict__ x, float* __restrict__ ws, int64_t cols,
                          int64_t rows, int64_t ns, const float* __restrict__ diag,
                          int64_t diag_stride, int64_t diag_len, double* __restrict__ flags) {
   __shared__ uint32_t s_hist[256];
   __shared__ uint32_t s_pick[2];
   __shared__ double s_red[SC_THREADS / 64];
-  // Columns are taken 64 to a wave, the workgroup's first wave only: the
-  // launch has one workgroup per 64 columns.
-  if ((int64_t)blockIdx.x * 64 < cols) {
-    const int64_t o = (int64_t)blockIdx.x * 64 + threadIdx.x;
-    if (threadIdx.x < 64 && o < cols)
-      scales[o] =
-          sqrtf(ordered_sum(ns, [&](int64_t s) { return ws[s * cols + o]; }) / (float)rows);
-    return;
+  int64_t b = blockIdx.x;
+  if (diag != nullptr) {
+    if (b == 0) {
+      const float skew = diagonal_skew(diag, diag_stride, diag_len, s_hist, s_pick, s_red);
+      if (threadIdx.x == 0) flags[1] = (double)skew;
+      return;
+    }
+    --b;
   }
-  const float skew = diagonal_skew(diag, diag_stride, diag_len, s_hist, s_pick, s_red);
-  if (threadIdx.x == 0) flags[1] = (double)skew;
+  const int64_t idx = b * SC_THREADS + threadIdx.x;
+  if (idx >= cols * ns) return;
+  const int64_t o = idx % cols, t0 = idx / cols * COL_SLICE;
+  const float* p = x + t0 * cols + o;
+  float slice = 0.0f;
+  if (t0 + COL_SLICE <= rows) {
+    float v[COL_SLICE];
+#pragma unroll
+    for (int t = 0; t < COL_SLICE; ++t) v[t] = p[t * cols];
+#pragma unroll
+    for (int t = 0; t < COL_SLICE; ++t) slice = slice + v[t] * v[t];
+  } else {
+    for (int64_t t = 0; t < rows - t0; ++t) {
+      const float v = p[t * cols];
+      slice = slice + v * v;
+    }
+  }
+  ws[idx] = slice;
 }
 
 // The output-channel scales of regularize (regularize.py:136-168) from the
@@ -1150,20 +1307,25 @@ int launch_hadamard(const float* in, float* out, int64_t rows, int64_t cols, int
   return check_launch(what);
 }
 
+// Whole 128 x 128 blocks of a matrix and the grid that takes one each.
+int block_grid(int64_t rows, int64_t cols, dim3* grid, const char* what) {
+  if (rows <= 0 || cols <= 0 || rows % HAD_N || cols % HAD_N)
+    return set_error("%s: both dimensions must be positive multiples of 128, got %lld x %lld",
+                     what, (long long)rows, (long long)cols);
+  if (cols / HAD_N > INT32_MAX || rows / HAD_N > 65535)
+    return set_error("%s: matrix too large", what);
+  *grid = dim3((unsigned)(cols / HAD_N), (unsigned)(rows / HAD_N));
+  return 0;
+}
+
 // Checks and grid of the unrotate kernel: whole 128 x 128 blocks, out and sv
 // read and written as float2.
 int unrotate_grid(const void* in, const float* su, const float* sv, const float* out,
                   int64_t rows, int64_t cols, dim3* grid, const char* what) {
   if (!in || !su || !sv || !out) return set_error("%s: NULL buffer", what);
-  if (rows <= 0 || cols <= 0 || rows % HAD_N || cols % HAD_N)
-    return set_error("%s: both dimensions must be positive multiples of 128, got %lld x %lld",
-                     what, (long long)rows, (long long)cols);
   if (((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(sv)) & 7) != 0)
     return set_error("%s: out and sv must be 8-byte aligned", what);
-  if (cols / HAD_N > INT32_MAX || rows / HAD_N > 65535)
-    return set_error("%s: matrix too large", what);
-  *grid = dim3((unsigned)(cols / HAD_N), (unsigned)(rows / HAD_N));
-  return 0;
+  return block_grid(rows, cols, grid, what);
 }
 
 }  // namespace
@@ -1183,6 +1345,29 @@ int exl3_hadamard128_scaled(const float* in, float* out, int64_t rows, int64_t c
     return set_error("hadamard128_scaled: slice sums of squares need side = 1");
   return launch_hadamard(in, out, rows, cols, side, divisor, slice_sumsq, stream,
                          "hadamard128_scaled");
+}
+
+int exl3_row_energy(const float* in, const float* sv, float* sums, int64_t rows, int64_t cols,
+                    void* stream) {
+  if (!in || !sv || !sums) return set_error("row_energy: NULL buffer");
+  dim3 grid;
+  if (block_grid(rows, cols, &grid, "row_energy")) return 1;
+  static_assert(HAD_N % EN_ROWS == 0, "whole workgroups to a row block");
+  unsigned b;
+  if (exl3::grid_1d(rows * (cols / HAD_N), EN_ROWS, &b, "row_energy")) return 1;
+  hipLaunchKernelGGL(row_energy_kernel, dim3(b), dim3(64 * EN_WAVES), 0, as_stream(stream), in,
+                     cols, sv, sums);
+  return check_launch("row_energy");
+}
+
+int exl3_rotate(const float* in, const float* sv, const float* su, float* out, int64_t rows,
+                int64_t cols, void* stream) {
+  if (!in || !sv || !su || !out) return set_error("rotate: NULL buffer");
+  dim3 grid;
+  if (block_grid(rows, cols, &grid, "rotate")) return 1;
+  hipLaunchKernelGGL(rotate_kernel, grid, dim3(RO_THREADS), 0, as_stream(stream), in, sv, su, out,
+                     cols);
+  return check_launch("rotate");
 }
 
 int exl3_unrotate(const float* in, const float* su, const float* sv, float* out, int64_t rows,
@@ -1245,7 +1430,6 @@ int exl3_output_scales(const float* x, int64_t rows, int64_t cols, const float* 
                        int64_t diag_stride, int64_t diag_len, const float* sv, int decide,
                        int forced, float* workspace, int64_t workspace_elems, float* scales,
                        float* divisor, float* sv_out, double* flags, void* stream) {
-  constexpr int bs = 32;
   if (!x || !sv || !workspace || !scales || !divisor || !sv_out || !flags)
     return set_error("output_scales: NULL buffer");
   if (rows <= 0 || cols <= 0) return set_error("output_scales: empty matrix");
@@ -1253,18 +1437,18 @@ int exl3_output_scales(const float* x, int64_t rows, int64_t cols, const float* 
   if (diag && (diag_len <= 0 || diag_len > INT32_MAX || diag_stride < 1))
     return set_error("output_scales: bad diagonal (%lld values, stride %lld)",
                      (long long)diag_len, (long long)diag_stride);
-  const int64_t ns = (rows + bs - 1) / bs;
+  const int64_t ns = (rows + COL_SLICE - 1) / COL_SLICE;
   if (workspace_elems < cols * ns)
     return set_error("output_scales: workspace holds %lld floats, %lld needed",
                      (long long)workspace_elems, (long long)(cols * ns));
   unsigned b1, b2;
-  if (exl3::grid_1d(cols * ns, 256, &b1, "output_scales")) return 1;
+  if (exl3::grid_1d(cols * ns, SC_THREADS, &b1, "output_scales")) return 1;
   if (exl3::grid_1d(cols, 64, &b2, "output_scales")) return 1;
   hipStream_t sm = as_stream(stream);
-  hipLaunchKernelGGL(block_rms_slices_kernel, dim3(b1), dim3(256), 0, sm, x, workspace, cols,
-                     rows, 1, cols, bs, ns, 0);
-  hipLaunchKernelGGL(column_scales_kernel, dim3(b2 + (diag ? 1 : 0)), dim3(SC_THREADS), 0, sm,
-                     workspace, scales, cols, rows, ns, diag, diag_stride, diag_len, flags);
+  hipLaunchKernelGGL(column_slices_kernel, dim3(b1 + (diag ? 1 : 0)), dim3(SC_THREADS), 0, sm, x,
+                     workspace, cols, rows, ns, diag, diag_stride, diag_len, flags);
+  hipLaunchKernelGGL(block_rms_reduce_columns_kernel, dim3(b2), dim3(64), 0, sm, workspace, scales,
+                     cols, rows, ns);
   hipLaunchKernelGGL(output_scales_kernel, dim3(1), dim3(SC_THREADS), 0, sm, scales, cols, sv,
                      decide, forced, divisor, sv_out, flags);
   return check_launch("output_scales");

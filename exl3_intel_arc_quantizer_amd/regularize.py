@@ -22,24 +22,23 @@ module makes three, on HIP kernels of ``libexl3_hip.so``:
 1. ``exl3_output_scales``: the column RMS of W, its mean, the skew of the
    Hessian diagonal (radix selection of its largest 2 %) and sv, every
    decision taken on the device;
-2. ``exl3_hadamard128_scaled`` side 1: W / sv and the right transform into a
-   new matrix in one read and one write, with the sums of squares of every
-   32-element row slice as a by-product; ``exl3_input_scales`` turns those
-   into the row RMS and su (a reduction over k x n/32 floats);
-3. ``exl3_hadamard128_scaled`` side 0: division by su and the left
-   transform, in place.
+2. ``exl3_row_energy``: the sums of squares of the rows of W / sv, which the
+   right transform keeps, in 128-element segments; ``exl3_input_scales``
+   turns those into the row RMS and su;
+3. ``exl3_rotate``: both divisions and both transforms of a 128 x 128 block in
+   one read and one write.
 
 The decisions (any energy, skew, scales applied) come back in one read after
-the last pass. A 4096 x 4096 weight takes 140 us, where torch operations on
+the last pass. A 4096 x 4096 weight takes 119 us, where torch operations on
 the scale vectors between the passes, a sort of the diagonal and strided
 reductions took 322 us.
 
 Rounding. Divisions are correctly rounded fp32, like torch's; the transform
-is the fast Walsh-Hadamard transform of ``exl3_hadamard128``. The RMS splits
-each row or column into 32-element slices and adds the slice sums in slice
-order, as the reference's ``block_rms`` does; within a slice the order is
-this build's (sequential for the column RMS, a butterfly over lanes for the
-row RMS), just as torch's own reduction order is an implementation detail.
+is the fast Walsh-Hadamard transform of ``exl3_hadamard128``. The column RMS
+sums 32-row slices in order and adds them in slice order, as the reference's
+``block_rms`` does; the row RMS adds the sums of 128-element segments in order,
+each a butterfly over lanes, and takes them before the orthonormal transform
+instead of after it, which leaves out the transform's roundings.
 Results therefore agree with the reference's to float32 rounding.
 """
 
@@ -149,7 +148,7 @@ def regularize(weight: torch.Tensor, su: torch.Tensor, sv: torch.Tensor,
     (regularize.py:83-211). ``weight`` is not modified. ``quant_args`` may
     force ``apply_out_scales``; when given, its ``zeros`` entry is set to
     whether W had no energy at all."""
-    from ._native import hadamard128_scaled, input_scales, output_scales
+    from ._native import input_scales, output_scales, rotate, row_energy
 
     _check_inputs(weight, su, sv, had_dim)
     k, n = weight.shape
@@ -177,18 +176,17 @@ def regularize(weight: torch.Tensor, su: torch.Tensor, sv: torch.Tensor,
     output_scales(w, sv, 2 if apply_out is None else int(apply_out), forced is not None,
                   out_scales, divisor, sv_out, flags, diag)
 
-    # Pass 2: W / sv and the right transform, with the row slice sums of
-    # squares for the input-channel scales.
-    work = torch.empty_like(w)
-    slice_sq = torch.empty((k, n // RMS_SLICE), **vec)
-    hadamard128_scaled(w, work, 1, divisor=divisor, slice_sumsq=slice_sq)
+    # Pass 2: the row sums of squares of W / sv (and so of its right
+    # transform, which is orthonormal) for the input-channel scales.
+    energy = torch.empty((k, n // HAD_DIM), **vec)
+    row_energy(w, divisor, energy)
     in_scales, su_out = torch.empty((k, 1), **vec), torch.empty((k, 1), **vec)
     su = su.to(device=dev, dtype=torch.float32).reshape(k).contiguous()
-    input_scales(slice_sq, su, in_scales, su_out, n)
-    del slice_sq
+    input_scales(energy, su, in_scales, su_out, n)
 
-    # Pass 3: divide by su and the left transform, in place.
-    hadamard128_scaled(work, work, 0, divisor=su_out)
+    # Pass 3: both divisions and both transforms.
+    work = torch.empty_like(w)
+    rotate(w, divisor, su_out, work)
 
     if skip_g_scale:
         g_scale = 1.0

@@ -41,6 +41,18 @@ int exl3_hadamard128(const float* in, float* out, int64_t rows, int64_t cols, in
 int exl3_hadamard128_scaled(const float* in, float* out, int64_t rows, int64_t cols, int side,
                             const float* divisor, float* slice_sumsq, void* stream);
 
+/* The two matrix passes of regularize (regularize.py:159-181) for a matrix of
+ * multiples of 128, each one read of `in`: sums[row * (cols / 128) + segment] =
+ * the sum of squares of every 128-element segment of the rows of (in / sv) H,
+ * and out = H (((in / sv) H) / su). H is orthonormal, so the sums are taken
+ * without it; out has the values of exl3_hadamard128_scaled side 1 (divisor
+ * sv) and then side 0 (divisor su). sv holds `cols` floats, su `rows`; out
+ * does not overlap in. */
+int exl3_row_energy(const float* in, const float* sv, float* sums, int64_t rows, int64_t cols,
+                    void* stream);
+int exl3_rotate(const float* in, const float* sv, const float* su, float* out, int64_t rows,
+                int64_t cols, void* stream);
+
 /* Replaces weight_from_quantized (hadamard.py:129-140): out = (H (in) * su)
  * H * sv with the blockwise transforms of exl3_hadamard128, su of `rows`
  * floats (one per row), sv of `cols` floats, in one pass over HBM; the same

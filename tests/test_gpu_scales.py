@@ -1,7 +1,8 @@
 """The scale kernels of regularize at the ends of their ranges: the skew by
 radix selection against a float64 sort (ties at the threshold, lengths
 around the 1/50 cut, a strided diagonal, NaN), the scale vectors against
-float64, and the row RMS at slice counts around the chunk and batch sizes."""
+float64, the row RMS at slice counts around the chunk and batch sizes, and the
+two passes over the matrix against the single transforms."""
 
 from __future__ import annotations
 
@@ -118,3 +119,42 @@ def test_row_reduction(rows, slices):
         np.testing.assert_allclose(out.cpu().numpy(),
                                    np.sqrt((x.cpu().numpy().astype(np.float64) ** 2).mean(0)),
                                    rtol=(36 + slices) * EPS32)
+
+
+@pytest.mark.parametrize("k,n", [(128, 128), (128, 1152), (640, 128), (384, 1024)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_rotation_passes(k, n, offset):
+    """The rotation is bit for bit the two scaled transforms and the row
+    energies are those of the first, also from a matrix that is only 4-byte
+    aligned; infinities and NaN land in the same places."""
+    import torch
+
+    from exl3_intel_arc_quantizer_amd._native import hadamard128_scaled, rotate, row_energy
+    g = torch.Generator(device="cuda").manual_seed(k + n)
+    x = torch.randn(k * n + offset, generator=g, device="cuda")[offset:].view(k, n)
+    sv = torch.rand(n, generator=g, device="cuda") * 3 + 0.1
+    su = torch.rand(k, generator=g, device="cuda") * 3 - 1.6
+    for special in (False, True):
+        if special:
+            x[1, 5], x[k - 1, n - 1], x[k // 2] = float("inf"), float("nan"), 0.0
+            x[6, 0] = x[6, 127] = float("-inf")
+            x[8, 64] = float("-inf")
+        before = x.clone()
+        mid, want = torch.empty(k, n, device="cuda"), torch.empty(k, n, device="cuda")
+        hadamard128_scaled(before, mid, 1, divisor=sv)
+        hadamard128_scaled(mid, want, 0, divisor=su)
+        out, energy = torch.empty_like(want), torch.empty(k, n // 128, device="cuda")
+        row_energy(x, sv, energy)
+        rotate(x, sv, su, out)
+        for got, ref in ((out, want), (x, before)):
+            assert torch.equal(got.isnan(), ref.isnan())
+            assert torch.equal(got.nan_to_num(), ref.nan_to_num())
+        wide = mid.double().square().view(k, n // 128, 128).sum(dim=2)
+        assert torch.equal(energy.isnan(), wide.isnan())
+        assert torch.equal(energy.isinf(), wide.isinf())
+        # A quotient, a square and seven additions here; seven additions, a
+        # scaling, and the quotient in the transform.
+        torch.testing.assert_close(energy.double().nan_to_num(posinf=0.0),
+                                   wide.nan_to_num(posinf=0.0), rtol=32 * EPS32, atol=0.0)
+    with pytest.raises(RuntimeError):
+        rotate(x, sv[:-1], su, out)
