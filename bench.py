@@ -99,7 +99,8 @@ ISA_CEILING = FLOP_PER_CANDIDATE / (1.25 * FLOP_PER_VALU_SLOT / 64)   # = 0.8
 LDS_BYTES_PER_CU_CLOCK = 128
 PEAK_LDS_TBPS = CUS * LDS_BYTES_PER_CU_CLOCK * NOMINAL_CLOCK_HZ / 1e12    # 78.6
 ENCODER_SOURCES = ("exl3_intel_arc_quantizer_amd/csrc/exl3_encoder.hip",
-                   "exl3_intel_arc_quantizer_amd/csrc/exl3_layout.h")
+                   "exl3_intel_arc_quantizer_amd/csrc/exl3_layout.h",
+                   "exl3_intel_arc_quantizer_amd/csrc/exl3_codebook.h")
 
 
 def encoder_source_sha() -> str:
