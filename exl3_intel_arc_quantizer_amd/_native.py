@@ -68,6 +68,8 @@ _SIGNATURES = {
     "exl3_cholesky_diag_block": (_c_int, [_c_vp, _c_i64, _c_int, _c_i64, _c_vp, _c_vp]),
     "exl3_gram": (_c_int, [_c_vp, _c_int, _c_i64, _c_i64, _c_i64, _c_float, _c_vp, _c_vp, _c_i64,
                            _c_vp]),
+    "exl3_gram_chunked": (_c_int, [_c_vp, _c_int, _c_i64, _c_i64, _c_i64, _c_float, _c_i64, _c_vp,
+                                   _c_vp, _c_i64, _c_vp]),
     "exl3_gram_workspace": (_c_i64, [_c_i64, _c_i64]),
     "exl3_damp_diagonal": (_c_int, [_c_vp, _c_i64, _c_i64, _c_double, _c_float, _c_vp, _c_vp]),
     "exl3_cholesky_block_order": (_c_int, []),
@@ -692,8 +694,9 @@ def gram_takes(x) -> bool:
             and x.data_ptr() % 16 == 0)
 
 
-def gram(x, scale: float):
-    """``scale * x.T @ x`` in float32 for bf16 / fp16 activations (exl3_gram)."""
+def gram(x, scale: float, chunk_tokens: int = 8192):
+    """``scale * x.T @ x`` in float32 for bf16 / fp16 activations, no float32
+    sum over more than ``chunk_tokens`` tokens (exl3_gram_chunked)."""
     torch = _torch()
     if not gram_takes(x):
         raise RuntimeError(f"gram does not take {x.dtype} {tuple(x.shape)} with strides "
@@ -705,9 +708,10 @@ def gram(x, scale: float):
         need = int(lib.exl3_gram_workspace(tokens, d))
         h = torch.empty((d, d), dtype=torch.float32, device=x.device)
         ws = torch.empty(max(need, 1), dtype=torch.float32, device=x.device)
-        _check(lib.exl3_gram(x.data_ptr(), int(x.dtype == torch.bfloat16), tokens, x.stride(0), d,
-                             float(scale), h.data_ptr(), ws.data_ptr(), ws.numel(),
-                             _stream(dev)), "gram")
+        _check(lib.exl3_gram_chunked(x.data_ptr(), int(x.dtype == torch.bfloat16), tokens,
+                                     x.stride(0), d, float(scale), min(chunk_tokens, tokens),
+                                     h.data_ptr(), ws.data_ptr(), ws.numel(), _stream(dev)),
+               "gram")
     return h
 
 

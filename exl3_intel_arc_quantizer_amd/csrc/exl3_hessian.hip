@@ -16,6 +16,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "../../include/exl3_layer.h"
 #include "exl3_errors.h"
@@ -68,11 +69,22 @@ __device__ __forceinline__ void lower_tile(int b, int& i, int& j) {
 // GPU to itself), of which the products are 0.48; the rest is staging and
 // LDS traffic. A library product of 8192 x 4096 bf16 activations took 262-300
 // us, and clearing, adding and dividing 60 more.
-template <int TS, bool BF16>
+//
+// An accumulator takes `run` chunks at most. A float32 sum loses up to half a
+// place of its total with every matrix instruction, so one accumulator over
+// all tokens loses in proportion to their number: 65,536 tokens x 4096, one
+// share, had a root mean square error of 1.26e-6 on the diagonal, where sums
+// over 8192 tokens, added in float32, have 1.6e-7. RUNS, for shares longer
+// than that: a run's sum is added to the tile's total, which its workgroup
+// alone reads and writes, in the partial tiles or, where there are none, in h
+// below the diagonal. That costs 7 % (8192 tokens a run: 65,536 x 4096 1337
+// us without it, 1431 with it, 16,384 x 4096 307 and 321); shorter shares,
+// which the loop around the runs made 1 % slower, take the kernel without it.
+template <int TS, bool BF16, bool RUNS>
 __global__ void __launch_bounds__(GR_THREADS, 2)
     gram_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_t tokens, int64_t d,
                 float scale, float* __restrict__ h, float* __restrict__ parts, int tiles,
-                int chunks, int share) {
+                int chunks, int share, int run) {
   constexpr int WI = TS / 32, WJ = TS / 64;          // 16 x 16 blocks of a wave
   constexpr int QP = TS / 8 + 2;                     // vectors of one column residue
   constexpr int OCT = 8 * QP;                        // vectors of one token octet
@@ -138,7 +150,7 @@ __global__ void __launch_bounds__(GR_THREADS, 2)
     }
   };
 
-  f32x4 acc[WI][WJ] = {};
+  f32x4 acc[WI][WJ];
   const int wi = (wave >> 2) * (TS / 2), wj = (wave & 3) * (TS / 4);
   auto vector_of = [&](int col) { return (col & 7) * QP + (col >> 3); };
   // Columns 16 apart are 2 vectors apart.
@@ -167,48 +179,96 @@ __global__ void __launch_bounds__(GR_THREADS, 2)
     }
   };
 
-  // The share's whole chunks, loads two chunks ahead of the products and no
-  // branch around them (past the end they repeat the last chunk), then the
-  // chunk that the tokens end in.
-  const int whole = (int64_t)c1 * GR_K <= tokens ? c1 : c1 - 1;
-  if (c0 < whole) {
-    const int last = whole - 1;
-    auto at = [&](int c) { return c < last ? c : last; };
-    fetch(c0, raw[0]);
-    fetch(at(c0 + 1), raw[1]);
-    stage(raw[0], 0);
-    __syncthreads();
-    int c = c0;
-    for (; c + 1 < whole; c += 2) {
-      fetch(at(c + 2), raw[0]);
-      multiply(0, [&] { stage(raw[1], 1); });
+  // The sum over chunks [r0, r1): the whole chunks, loads two chunks ahead of
+  // the products and no branch around them (past the end they repeat the last
+  // chunk), then the chunk that the tokens end in.
+  auto sum_run = [&](int r0, int r1) {
+#pragma unroll
+    for (int p = 0; p < WI; ++p) {
+#pragma unroll
+      for (int q = 0; q < WJ; ++q) acc[p][q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    const int whole = (int64_t)r1 * GR_K <= tokens ? r1 : r1 - 1;
+    if (r0 < whole) {
+      const int last = whole - 1;
+      auto at = [&](int c) { return c < last ? c : last; };
+      fetch(r0, raw[0]);
+      fetch(at(r0 + 1), raw[1]);
+      stage(raw[0], 0);
       __syncthreads();
-      fetch(at(c + 3), raw[1]);
-      multiply(1, [&] { stage(raw[0], 0); });
+      int c = r0;
+      for (; c + 1 < whole; c += 2) {
+        fetch(at(c + 2), raw[0]);
+        multiply(0, [&] { stage(raw[1], 1); });
+        __syncthreads();
+        fetch(at(c + 3), raw[1]);
+        multiply(1, [&] { stage(raw[0], 0); });
+        __syncthreads();
+      }
+      if (c < whole) multiply(0, [] {});
       __syncthreads();
     }
-    if (c < whole) multiply(0, [] {});
-    __syncthreads();
-  }
-  if (whole < c1) {
-    fetch_end(whole, raw[0]);
-    stage(raw[0], 0);
-    __syncthreads();
-    multiply(0, [] {});
+    if (whole < r1) {
+      fetch_end(whole, raw[0]);
+      stage(raw[0], 0);
+      __syncthreads();
+      multiply(0, [] {});
+      if constexpr (RUNS) __syncthreads();
+    }
+  };
+
+  // Lane l holds rows 4 (l / 16) + t of column l % 16 of a block in element
+  // t; d is a multiple of 8, so a lane's four rows are in the matrix or past
+  // it together.
+  const int row0 = wi + 4 * (lane >> 4), col0 = wj + (lane & 15);
+  auto inside = [&](int p, int q) { return i0 + row0 + 16 * p < d && j0 + col0 + 16 * q < d; };
+  if constexpr (!RUNS) {
+    sum_run(c0, c1);
+  } else {
+    auto with_total = [&](auto f) {
+      float* total = parts ? parts + (int64_t)blockIdx.x * TS * TS : h + i0 * d + j0;
+      int64_t ld = parts ? TS : d;
+      // Not known to be the same in every run: the addresses of 4 WI WJ
+      // elements would otherwise stay in registers through the products.
+      asm volatile("" : "+s"(total), "+s"(ld));
+      float* own = total + row0 * ld + col0;
+#pragma unroll
+      for (int p = 0; p < WI; ++p) {
+#pragma unroll
+        for (int q = 0; q < WJ; ++q) {
+          if (parts || inside(p, q)) f(own + 16 * p * ld + 16 * q, ld, acc[p][q]);
+        }
+      }
+    };
+    for (int r0 = c0;;) {
+      const int r1 = c1 - r0 > run ? r0 + run : c1;
+      sum_run(r0, r1);
+      if (r0 > c0)
+        with_total([](const float* total, int64_t ld, f32x4& sum) {
+          f32x4 v;
+#pragma unroll
+          for (int t = 0; t < 4; ++t) v[t] = total[t * ld];
+          sum = v + sum;
+        });
+      r0 = r1;
+      if (r0 >= c1) break;
+      with_total([](float* total, int64_t ld, const f32x4& sum) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) total[t * ld] = sum[t];
+      });
+    }
   }
 
-  // Lane l holds rows 4 (l / 16) + t of column l % 16 of a block in element t.
   float* part = parts ? parts + (int64_t)blockIdx.x * TS * TS : nullptr;
 #pragma unroll
   for (int p = 0; p < WI; ++p) {
 #pragma unroll
     for (int q = 0; q < WJ; ++q) {
-      const int col = wj + 16 * q + (lane & 15);
-      const int row = wi + 16 * p + 4 * (lane >> 4);
+      const int col = col0 + 16 * q, row = row0 + 16 * p;
       if (part) {
 #pragma unroll
         for (int t = 0; t < 4; ++t) part[(row + t) * TS + col] = acc[p][q][t];
-      } else if (j0 + col < d && i0 + row < d) {  // d is a multiple of 8
+      } else if (inside(p, q)) {
 #pragma unroll
         for (int t = 0; t < 4; ++t) h[(i0 + row + t) * d + j0 + col] = acc[p][q][t] * scale;
         if (ti != tj) {
@@ -336,11 +396,20 @@ int64_t exl3_gram_workspace(int64_t tokens, int64_t d) {
 
 int exl3_gram(const uint16_t* x, int bf16, int64_t tokens, int64_t ldx, int64_t d, float scale,
               float* h, float* workspace, int64_t workspace_elems, void* stream) {
+  return exl3_gram_chunked(x, bf16, tokens, ldx, d, scale, 8192, h, workspace, workspace_elems,
+                           stream);
+}
+
+int exl3_gram_chunked(const uint16_t* x, int bf16, int64_t tokens, int64_t ldx, int64_t d,
+                      float scale, int64_t chunk_tokens, float* h, float* workspace,
+                      int64_t workspace_elems, void* stream) {
   if (!x || !h) return set_error("gram: NULL buffer");
   if (!gram_shape_ok(tokens, d) || ldx < d || ldx % 8 || ldx > 1 << 24)
     return set_error("gram: bad shape (%lld tokens, d %lld, row stride %lld)", (long long)tokens,
                      (long long)d, (long long)ldx);
   if (reinterpret_cast<uintptr_t>(x) & 15) return set_error("gram: x must be 16-byte aligned");
+  if (chunk_tokens < 1)
+    return set_error("gram: chunk_tokens must be positive, got %lld", (long long)chunk_tokens);
   const GramPlan p = gram_plan(tokens, d, current_cus());
   const int64_t need = p.splits > 1 ? (int64_t)p.splits * p.tiles * p.ts * p.ts : 0;
   if (need && (!workspace || workspace_elems < need))
@@ -348,17 +417,24 @@ int exl3_gram(const uint16_t* x, int bf16, int64_t tokens, int64_t ldx, int64_t 
                      (long long)(workspace ? workspace_elems : 0), (long long)need);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   float* parts = need ? workspace : nullptr;
+  // Whole chunks of the kernel, at least one; all of them for one sum.
+  const int run = chunk_tokens >= tokens
+                      ? p.chunks
+                      : (int)std::clamp<int64_t>(chunk_tokens / GR_K, 1, p.chunks);
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)(p.tiles * p.splits)), dim3(GR_THREADS), 0, st, x,
-                       ldx, tokens, d, scale, h, parts, p.tiles, p.chunks, p.share);
+                       ldx, tokens, d, scale, h, parts, p.tiles, p.chunks, p.share, run);
   };
-  if (p.ts == 192) {
-    if (bf16) launch(gram_kernel<192, true>);
-    else launch(gram_kernel<192, false>);
-  } else {
-    if (bf16) launch(gram_kernel<128, true>);
-    else launch(gram_kernel<128, false>);
-  }
+  auto launch_tile = [&](auto side, auto runs) {
+    if (bf16) launch(gram_kernel<side(), true, runs()>);
+    else launch(gram_kernel<side(), false, runs()>);
+  };
+  auto launch_runs = [&](auto runs) {
+    if (p.ts == 192) launch_tile(std::integral_constant<int, 192>{}, runs);
+    else launch_tile(std::integral_constant<int, 128>{}, runs);
+  };
+  if (p.share > run) launch_runs(std::true_type{});
+  else launch_runs(std::false_type{});
   if (parts)
     hipLaunchKernelGGL(gram_reduce_kernel, dim3((unsigned)p.tiles, (p.ts / 32) * (p.ts / 32)),
                        dim3(256), 0, st, parts, p.ts, p.tiles, p.splits, scale, h, d);

@@ -52,7 +52,8 @@ def hessian_from_activations(x: torch.Tensor, damping_lambda: float = DEFAULT_DA
     bf16 / fp16 activations on the GPU go straight onto the matrix cores
     (``exl3_gram``): their products are exact in float32, so the result is
     the float32 product of the converted values up to summation order, of
-    which only the lower triangle is computed. Layouts that kernel does not
+    which only the lower triangle is computed, the chunks' sums added in
+    float32 as on the other paths. Layouts that kernel does not
     take (an odd width, strided columns) go through a half-precision GEMM
     with float32 output, float32 activations through a float32 GEMM. On the
     GPU the damping and the floor are one launch, and the mean that the
@@ -65,7 +66,7 @@ def hessian_from_activations(x: torch.Tensor, damping_lambda: float = DEFAULT_DA
     # The kernels record no gradient.
     native = flat.device.type == "cuda" and not (torch.is_grad_enabled() and x.requires_grad)
     if native and half and len(starts) > 0 and gram_takes(flat):
-        H = gram(flat, 1.0 / tokens)
+        H = gram(flat, 1.0 / tokens, chunk_tokens)
     else:
         H = None
         for s in starts:

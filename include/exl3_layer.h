@@ -102,8 +102,14 @@ int exl3_output_scales(const float* x, int64_t rows, int64_t cols, const float* 
  * X^T X for X of `tokens` rows (row stride ldx elements) and d columns, bf16
  * (bf16 != 0) or fp16, products and sums in float32, h float32 d x d
  * contiguous and exactly symmetric. d and ldx are multiples of 8, x is
- * 16-byte aligned. workspace: exl3_gram_workspace floats (0 where the tokens
- * are not shared out). */
+ * 16-byte aligned. No float32 sum runs over more than chunk_tokens tokens
+ * (>= 1; taken down to a multiple of 64, or 64): the chunks' sums are added
+ * in float32, in token order. exl3_gram is exl3_gram_chunked with 8192.
+ * workspace: exl3_gram_workspace floats (0 where the tokens are not shared
+ * out). */
+int exl3_gram_chunked(const uint16_t* x, int bf16, int64_t tokens, int64_t ldx, int64_t d,
+                      float scale, int64_t chunk_tokens, float* h, float* workspace,
+                      int64_t workspace_elems, void* stream);
 int exl3_gram(const uint16_t* x, int bf16, int64_t tokens, int64_t ldx, int64_t d, float scale,
               float* h, float* workspace, int64_t workspace_elems, void* stream);
 

@@ -71,3 +71,99 @@ def test_layouts_of_hessian_from_activations():
         assert float((h.double() - want).norm() / want.norm()) < 1e-6
     with pytest.raises(ValueError):
         hessian_from_activations(x[..., :256].contiguous(), chunk_tokens=0)
+
+
+@pytest.mark.parametrize("tokens,d", [(65536, 4096), (70001, 4096), (131072, 2048)])
+def test_long_sums_are_no_worse_than_chunked_ones(tokens, d):
+    """The error against float64 is that of float32 sums over at most 8192
+    tokens, added in float32, whatever the token count and the width's share
+    of the GPU: the diagonal (growing sums) and the rest."""
+    import torch
+
+    from exl3_intel_arc_quantizer_amd.layer_quant import hessian_from_activations
+    g = torch.Generator(device="cuda").manual_seed(d)
+    x = torch.randn(tokens, d, generator=g, device="cuda").to(torch.bfloat16)
+    chunked = torch.zeros(d, d, device="cuda")
+    want = torch.zeros(d, d, dtype=torch.float64, device="cuda")
+    for s in range(0, tokens, 8192):
+        part = x[s:s + 8192]
+        chunked += torch.mm(part.T, part, out_dtype=torch.float32)
+        wide = part.double()
+        want += wide.T @ wide
+    chunked /= tokens
+    want /= tokens
+    # The damping, here 1e-8, is far below a rounding of the diagonal (1).
+    h, _ = hessian_from_activations(x, damping_lambda=0.0, zero_floor=0.0)
+    eye = torch.eye(d, dtype=torch.bool, device="cuda")
+    for mask in (eye, ~eye):
+        # As many roundings in another order: 1.25 for the spread of a root
+        # mean square over thousands of entries.
+        ours, theirs = (float((v.double() - want)[mask].square().mean().sqrt())
+                        for v in (h, chunked))
+        assert ours <= 1.25 * theirs, (ours, theirs)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("d", [8, 4096])
+def test_chunk_tokens_have_sums_of_their_own(d, dtype):
+    """2^30 from the first token swallows products of 1 (its last place is
+    128), but not the sums that chunks of 1024 tokens bring: one float32
+    sum over all tokens would stay at 2^30."""
+    import torch
+
+    from exl3_intel_arc_quantizer_amd.layer_quant import hessian_from_activations
+    x = torch.ones(4096, d, device="cuda", dtype=getattr(torch, dtype))
+    x[0] = 2.0 ** 15
+    h, damp = hessian_from_activations(x, damping_lambda=0.0, chunk_tokens=1024)
+    assert damp == 1e-8
+    exact = 2.0 ** 30 + 4095.0
+    # The first chunk may lose its other 1023 tokens; a half rounding (64) for
+    # each of the three additions.
+    assert bool(((h.double() * 4096 - exact).abs() <= 1023 + 3 * 64).all())
+
+
+@pytest.mark.parametrize("tokens,d,chunk", [(64, 136, 64), (129, 136, 64), (1000, 520, 100),
+                                            (4097, 328, 192), (2000, 4096, 640), (700, 4096, 1)])
+def test_chunk_edges(tokens, d, chunk):
+    """Chunks that end inside and at the ends of shares, a ragged last one,
+    lengths that are no multiple of the kernel's 64 tokens."""
+    import torch
+
+    from exl3_intel_arc_quantizer_amd.layer_quant import hessian_from_activations
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    x = torch.randn(tokens, d, generator=g, device="cuda").to(torch.bfloat16)
+    wide = x.double()
+    h, damp = hessian_from_activations(x, zero_floor=0.0, chunk_tokens=chunk)
+    assert torch.equal(h, h.T)
+    h = h.double()
+    h.diagonal().sub_(damp)
+    # Each sum of `tokens` exact products rounds at most that often at the
+    # size of the sum of magnitudes, and at the division and the damping.
+    bound = (wide.abs().T @ wide.abs()) / tokens * (tokens + 4) * 2.0 ** -24
+    assert bool(((h - wide.T @ wide / tokens).abs() <= bound + 1e-7 * damp).all())
+
+
+def test_two_rounds_of_workgroups():
+    """A width whose tiles (378) are more than the GPU's compute units."""
+    import torch
+
+    from exl3_intel_arc_quantizer_amd._native import gram
+    x = torch.randn(300, 5000, device="cuda").to(torch.bfloat16)
+    h, wide = gram(x, 1.0), x.double()
+    assert torch.equal(h, h.T)
+    bound = (wide.abs().T @ wide.abs()) * 302 * 2.0 ** -24
+    assert bool(((h.double() - wide.T @ wide).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("width", [260, 255])
+def test_chunks_of_other_layouts(width):
+    import torch
+
+    from exl3_intel_arc_quantizer_amd._native import gram_takes
+    from exl3_intel_arc_quantizer_amd.layer_quant import hessian_from_activations
+    x = torch.randn(900, 264, device="cuda").to(torch.bfloat16)[:, :width]
+    assert not gram_takes(x)
+    h, damp = hessian_from_activations(x, chunk_tokens=256)     # three and a part
+    want = x.double().T @ x.double() / 900
+    want.diagonal().add_(damp)
+    assert float((h.double() - want).norm() / want.norm()) < 1e-6
