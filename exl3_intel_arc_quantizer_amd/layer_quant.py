@@ -76,7 +76,8 @@ def hessian_from_activations(x: torch.Tensor, damping_lambda: float = DEFAULT_DA
             else:
                 xf = xc.to(torch.float32)
                 part = xf.T @ xf
-            H = part if H is None else H.add_(part)
+            # Under autocast a product may be narrower; the sum is not.
+            H = part.to(torch.float32) if H is None else H.add_(part)
         if H is None:
             H = torch.zeros((d, d), dtype=torch.float32, device=x.device)
         H /= max(1, tokens)

@@ -167,3 +167,25 @@ def test_chunks_of_other_layouts(width):
     want = x.double().T @ x.double() / 900
     want.diagonal().add_(damp)
     assert float((h.double() - want).norm() / want.norm()) < 1e-6
+
+
+def test_float32_sums_under_autocast():
+    """Autocast chooses the products' precision, never the sum's, which is
+    what the damping and the caller take."""
+    import torch
+
+    from exl3_intel_arc_quantizer_amd.layer_quant import hessian_from_activations
+    x = torch.randn(900, 256, device="cuda")
+
+    def error(h, damp, x):
+        assert h.dtype == torch.float32
+        want = x.double().T @ x.double() / 900
+        want.diagonal().add_(damp)
+        return float((h.double() - want).norm() / want.norm())
+
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        for chunk in (256, 8192):
+            # Inputs and products rounded to 8 bits.
+            assert error(*hessian_from_activations(x, chunk_tokens=chunk), x) < 3 * 2.0 ** -8
+        half = x.to(torch.float16)      # products in float32 there, autocast or not
+        assert error(*hessian_from_activations(half), half) < 1e-6
