@@ -17,9 +17,10 @@ from __future__ import annotations
 
 import functools
 import math
-from typing import Optional
+from typing import Callable, Optional
 
 import torch
+from torch.autograd import forward_ad
 
 HAD_DIM = 128
 
@@ -112,6 +113,54 @@ def blockwise_preapply_had_r_(x: torch.Tensor, had_dim: int = HAD_DIM) -> torch.
     return _in_place(x, 1, had_dim)
 
 
+def records(t: torch.Tensor) -> bool:
+    """Whether torch follows operations on ``t``, for a backward pass or for
+    the tangent of a forward-mode (dual) tensor. The kernels record nothing."""
+    if t.requires_grad and torch.is_grad_enabled():
+        return True
+    # Tangents exist inside a dual level only; asking for the level first
+    # saves a microsecond of a call that takes 40.
+    return getattr(forward_ad, "_current_level", 0) >= 0 and \
+        forward_ad.unpack_dual(t).tangent is not None
+
+
+class _RowScaled(torch.autograd.Function):
+    """``transform(su)`` = (H_l w * su) H_r, whose derivatives in su need the
+    rows H_l w: those of su = 1, the right transform undone."""
+
+    @staticmethod
+    def forward(ctx, su: torch.Tensor, transform: Callable) -> torch.Tensor:
+        rows = _had128(transform(torch.ones_like(su)), 1, HAD_DIM, None)
+        ctx.save_for_backward(rows)
+        ctx.save_for_forward(rows)
+        return transform(su)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, grad: torch.Tensor) -> tuple:
+        rows, = ctx.saved_tensors
+        return (_had128(grad, 1, HAD_DIM, None) * rows).sum(dim=1), None
+
+    @staticmethod
+    def jvp(ctx, tangent: torch.Tensor, _) -> torch.Tensor:
+        rows, = ctx.saved_tensors
+        return _had128(rows * tangent[:, None], 1, HAD_DIM, None)
+
+
+def with_scales(transform: Callable, su: torch.Tensor, sv: torch.Tensor) -> torch.Tensor:
+    """``transform(su, sv)`` = ((H_l w * su) H_r) * sv, a kernel into a new
+    tensor, with the gradients and tangents of su and sv where torch follows
+    them: the last product is then torch's (the kernel's x 1 is exact)."""
+    if not (records(su) or records(sv)):
+        return transform(su, sv)
+    ones = torch.ones_like(sv)
+
+    def rows_only(v: torch.Tensor) -> torch.Tensor:
+        return transform(v, ones)
+
+    return (_RowScaled.apply(su, rows_only) if records(su) else rows_only(su)) * sv
+
+
 def scale_vectors(su: torch.Tensor, sv: torch.Tensor, k: int, n: int,
                   device: torch.device) -> tuple:
     """su and sv as float32 vectors on ``device``, sv 8-byte aligned."""
@@ -135,10 +184,10 @@ def weight_from_quantized(w_hat: torch.Tensor, su: torch.Tensor,
     work = w_hat if (w_hat.dtype == torch.float32 and w_hat.is_contiguous()) else \
         w_hat.to(torch.float32).contiguous()
     su, sv = scale_vectors(su, sv, k, n, work.device)
-    out = torch.empty_like(work)
-    if torch.is_grad_enabled() and sv.requires_grad:
-        # The last step is then torch's, which records sv's gradient; x 1 is exact.
-        unrotate(work, su, torch.ones_like(sv), out)
-        return out * sv
-    unrotate(work, su, sv, out)
-    return out
+
+    def transform(su: torch.Tensor, sv: torch.Tensor) -> torch.Tensor:
+        out = torch.empty_like(work)
+        unrotate(work, su, sv, out)
+        return out
+
+    return with_scales(transform, su, sv)

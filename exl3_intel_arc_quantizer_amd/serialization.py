@@ -21,7 +21,7 @@ from typing import Any, Dict, Optional, Tuple, Union
 
 import torch
 
-from .hadamard import HAD_DIM, scale_vectors
+from .hadamard import HAD_DIM, scale_vectors, with_scales
 from .trellis_format import CB_3INST, CB_MCG, CB_MUL1
 
 __all__ = ["pack_module_trellis", "unpack_module_trellis", "decode_weight_from_storage",
@@ -96,13 +96,13 @@ def decode_weight_from_storage(trellis: torch.Tensor, suh: torch.Tensor, svh: to
     if packed.data_ptr() % 4:
         packed = packed.clone()
     su, sv = scale_vectors(suh, svh, k, n, packed.device)
-    w = torch.empty((k, n), dtype=torch.float32, device=packed.device)
-    if torch.is_grad_enabled() and sv.requires_grad:
-        # The last step is then torch's, which records svh's gradient; x 1 is exact.
-        decode_weight(packed, su, torch.ones_like(sv), w, K, cb)
-        return (w * sv).to(trellis.device)
-    decode_weight(packed, su, sv, w, K, cb)
-    return w.to(trellis.device)
+
+    def transform(su: torch.Tensor, sv: torch.Tensor) -> torch.Tensor:
+        w = torch.empty((k, n), dtype=torch.float32, device=packed.device)
+        decode_weight(packed, su, sv, w, K, cb)
+        return w
+
+    return with_scales(transform, su, sv).to(trellis.device)
 
 
 def build_layer_tensors(module_results: Dict[str, Any], layer_idx: int = 0,

@@ -101,3 +101,62 @@ def test_gradient_of_output_scales():
         # Sums of 128 float32 terms.
         want, size = (plain.double() / sv).sum(dim=0), (plain.double() / sv).abs().sum(dim=0)
         assert bool(((leaf.grad - want).abs() <= 140 * 2.0 ** -24 * size).all())
+
+
+def _decoders(torch, g):
+    from exl3_intel_arc_quantizer_amd.hadamard import weight_from_quantized
+    from exl3_intel_arc_quantizer_amd.serialization import (decode_weight_from_storage,
+                                                            pack_module_trellis)
+    w = torch.randn(128, 256, generator=g, device="cuda")
+    states = torch.randint(-32768, 32768, (8, 16, 256), generator=g, device="cuda",
+                           dtype=torch.int32).to(torch.int16)
+    trellis = pack_module_trellis(states, 4)
+    return (lambda su, sv: weight_from_quantized(w, su, sv),
+            lambda su, sv: decode_weight_from_storage(trellis, su, sv, 4))
+
+
+def test_tangent_of_output_scales():
+    """A forward-mode sv gives the same weight and carries its tangent."""
+    import torch
+    import torch.autograd.forward_ad as forward_ad
+    g = torch.Generator(device="cuda").manual_seed(6)
+    su, sv, t = (torch.rand(n, generator=g, device="cuda") + 0.5 for n in (128, 256, 256))
+    for decode in _decoders(torch, g):
+        plain = decode(su, sv)
+        with forward_ad.dual_level():
+            out, tangent = forward_ad.unpack_dual(decode(su, forward_ad.make_dual(sv, t)))
+            assert torch.equal(out, plain) and tangent is not None
+            # One product an element, one rounding; the weight's own is one more.
+            torch.testing.assert_close(tangent.double(), plain.double() / sv * t,
+                                       rtol=4 * 2.0 ** -24, atol=0.0)
+
+
+def test_derivatives_of_input_scales():
+    """A recorded or forward-mode su, alone or beside a recorded sv, gives the
+    same weight, and its derivatives are those of a product that is linear in
+    su."""
+    import torch
+    import torch.autograd.forward_ad as forward_ad
+    g = torch.Generator(device="cuda").manual_seed(7)
+    su, sv, t = (torch.rand(n, generator=g, device="cuda") + 0.5 for n in (128, 256, 128))
+    pull = torch.randn(128, 256, generator=g, device="cuda")
+    for decode in _decoders(torch, g):
+        plain = decode(su, sv)
+        # d/d su[r] of sum(pull * weight): row r of a weight with su = 1.
+        rows = decode(torch.ones_like(su), sv).double() * pull.double()
+        for with_sv in (False, True):
+            leaf = su.clone().requires_grad_()
+            col = sv.clone().requires_grad_(with_sv)
+            out = decode(leaf, col)
+            assert torch.equal(out, plain)
+            out.backward(pull)
+            # 256 products a sum, behind three transforms of 7 levels.
+            size = decode(torch.ones_like(su), sv).double().norm(dim=1) * pull.double().norm(dim=1)
+            err = (leaf.grad.double() - rows.sum(dim=1)).abs()
+            assert bool((err <= 64 * 2.0 ** -24 * size).all()), float((err / size).max())
+            assert (col.grad is not None) == with_sv
+        with forward_ad.dual_level():
+            out, tangent = forward_ad.unpack_dual(decode(forward_ad.make_dual(su, t), sv))
+            assert torch.equal(out, plain)
+            want = decode(t, sv).double()
+            assert float((tangent.double() - want).norm() / want.norm()) < 64 * 2.0 ** -24
