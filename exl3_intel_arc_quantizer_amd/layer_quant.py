@@ -26,7 +26,7 @@ from typing import Dict, List, Optional, Tuple
 import torch
 
 from ._native import damp_diagonal, gram, gram_takes
-from .hadamard import HAD_DIM, blockwise_preapply_had_l_, blockwise_preapply_had_r_, \
+from .hadamard import HAD_DIM, blockwise_preapply_had_l_, blockwise_preapply_had_r_, records, \
     weight_from_quantized
 from .ldlq import (DEFAULT_BLOCK_SIZE, DEFAULT_BUF_SIZE_K, BlockLDLResult, LDLQResult,
                    block_ldl, ldlq, ldlq_lockstep)
@@ -63,8 +63,7 @@ def hessian_from_activations(x: torch.Tensor, damping_lambda: float = DEFAULT_DA
     tokens = flat.shape[0]
     starts = range(0, tokens, chunk_tokens)
     half = flat.device.type == "cuda" and flat.dtype in (torch.bfloat16, torch.float16)
-    # The kernels record no gradient.
-    native = flat.device.type == "cuda" and not (torch.is_grad_enabled() and x.requires_grad)
+    native = flat.device.type == "cuda" and not records(x)
     if native and half and len(starts) > 0 and gram_takes(flat):
         H = gram(flat, 1.0 / tokens, chunk_tokens)
     else:

@@ -189,3 +189,27 @@ def test_float32_sums_under_autocast():
             assert error(*hessian_from_activations(x, chunk_tokens=chunk), x) < 3 * 2.0 ** -8
         half = x.to(torch.float16)      # products in float32 there, autocast or not
         assert error(*hessian_from_activations(half), half) < 1e-6
+
+
+def test_followed_activations():
+    """Activations that torch follows go through torch's products: float32
+    ones carry gradients and tangents, half-precision ones, whose products
+    have no derivatives, are refused and not passed on without them."""
+    import torch
+    import torch.autograd.forward_ad as forward_ad
+
+    from exl3_intel_arc_quantizer_amd.layer_quant import hessian_from_activations
+    x = torch.randn(300, 128, device="cuda")
+    t = torch.randn(300, 128, device="cuda")
+    cross = x.double().T @ t.double() / 300
+    with forward_ad.dual_level():
+        h, _ = hessian_from_activations(forward_ad.make_dual(x, t))
+        tangent = forward_ad.unpack_dual(h).tangent.double()
+        assert float((tangent - cross - cross.T).norm() / cross.norm()) < 1e-5
+        with pytest.raises((NotImplementedError, RuntimeError)):
+            hessian_from_activations(forward_ad.make_dual(x.bfloat16(), t.bfloat16()))
+    leaf = x.clone().requires_grad_()
+    h, _ = hessian_from_activations(leaf)
+    h.sum().backward()
+    want = 2.0 * x.double().sum(dim=1, keepdim=True).expand(-1, 128) / 300
+    assert float((leaf.grad.double() - want).norm() / want.norm()) < 1e-5
