@@ -49,7 +49,7 @@ from typing import Callable, Optional, Tuple
 
 import torch
 
-from .hadamard import HAD_DIM
+from .hadamard import HAD_DIM, records
 
 # The kernels of exl3_output_scales / exl3_input_scales carry these values.
 CODEBOOK_SCALE = 1.24371088     # the codebook's RMS, regularize.py:33
@@ -173,8 +173,18 @@ def regularize(weight: torch.Tensor, su: torch.Tensor, sv: torch.Tensor,
             diag = H_diag
         else:
             flags[1] = _skew_tensor(H_diag)
-    output_scales(w, sv, 2 if apply_out is None else int(apply_out), forced is not None,
+    # Where torch follows sv, the kernel works on ones and sv is folded by
+    # torch's operations, to the same values.
+    follow_sv = records(sv)
+    output_scales(w, torch.ones_like(sv) if follow_sv else sv,
+                  2 if apply_out is None else int(apply_out), forced is not None,
                   out_scales, divisor, sv_out, flags, diag)
+    if follow_sv:
+        dead_cols = sv_out == 0.0
+        sv = sv.reshape(1, n)
+        sv_out = torch.where(flags[2] != 0.0, (sv * out_scales + EPS).float(), sv)
+        divisor = sv_out.detach().reshape(n).clone()
+        sv_out = sv_out.masked_fill(dead_cols, 0.0)
 
     # Pass 2: the row sums of squares of W / sv (and so of its right
     # transform, which is orthonormal) for the input-channel scales.
@@ -183,6 +193,8 @@ def regularize(weight: torch.Tensor, su: torch.Tensor, sv: torch.Tensor,
     in_scales, su_out = torch.empty((k, 1), **vec), torch.empty((k, 1), **vec)
     su = su.to(device=dev, dtype=torch.float32).reshape(k).contiguous()
     input_scales(energy, su, in_scales, su_out, n)
+    if records(su):
+        su_out = (su.reshape(k, 1) * in_scales / (-CODEBOOK_SCALE) + EPS).float()
 
     # Pass 3: both divisions and both transforms.
     work = torch.empty_like(w)

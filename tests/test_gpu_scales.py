@@ -158,3 +158,56 @@ def test_rotation_passes(k, n, offset):
                                    wide.nan_to_num(posinf=0.0), rtol=32 * EPS32, atol=0.0)
     with pytest.raises(RuntimeError):
         rotate(x, sv[:-1], su, out)
+
+
+@pytest.mark.parametrize("apply", [None, False, True])
+@pytest.mark.parametrize("skewed", [False, True])
+def test_recorded_scales(apply, skewed):
+    """regularize's su and sv keep the gradient and the tangent of those given:
+    both are affine in what they come from (regularize.py:159-181), at the same
+    values as without."""
+    import torch
+    import torch.autograd.forward_ad as forward_ad
+
+    from exl3_intel_arc_quantizer_amd.regularize import regularize
+    k, n = 256, 384
+    g = torch.Generator(device="cuda").manual_seed(9)
+    w = torch.randn(k, n, generator=g, device="cuda")
+    w[:, 7] = 0.0
+    w[9] = 0.0
+    su = torch.rand(k, 1, generator=g, device="cuda") + 0.5
+    sv = torch.rand(1, n, generator=g, device="cuda") + 0.5
+    sv[0, 3] = 0.1
+    diag = torch.rand(k, generator=g, device="cuda") + 0.1
+    if skewed:
+        diag[:2] = 1e6
+    args = lambda: None if apply is None else {"apply_out_scales": apply}
+    plain = regularize(w, su, sv, quant_args=args(), H_diag=diag)
+    assert not plain.su.requires_grad and not plain.sv.requires_grad
+    a, b = su.clone().requires_grad_(), sv.clone().requires_grad_()
+    for pair in ((a, sv), (su, b), (a, b)):
+        a.grad = b.grad = None
+        r = regularize(w, *pair, quant_args=args(), H_diag=diag)
+        for name in ("weight", "su", "sv", "out_channel_scales", "in_channel_scales"):
+            assert torch.equal(getattr(r, name), getattr(plain, name)), name
+        assert r.apply_out_scales == plain.apply_out_scales
+        assert r.su.requires_grad == pair[0].requires_grad
+        assert r.sv.requires_grad == pair[1].requires_grad and not r.weight.requires_grad
+        (r.su.sum() + r.sv.sum()).backward() if r.su.requires_grad and r.sv.requires_grad else \
+            (r.su if r.su.requires_grad else r.sv).sum().backward()
+        if r.su.requires_grad:
+            torch.testing.assert_close(a.grad, plain.in_channel_scales / -1.24371088,
+                                       rtol=4 * EPS32, atol=0.0)
+        if r.sv.requires_grad:
+            want = plain.out_channel_scales.clone() if plain.apply_out_scales \
+                else torch.ones_like(sv)
+            want[0, 7] = 0.0
+            torch.testing.assert_close(b.grad, want, rtol=4 * EPS32, atol=0.0)
+    with forward_ad.dual_level():
+        r = regularize(w, forward_ad.make_dual(su, 2 * su), forward_ad.make_dual(sv, 3 * sv),
+                       quant_args=args(), H_diag=diag)
+        (s0, st), (v0, vt) = (forward_ad.unpack_dual(x) for x in (r.su, r.sv))
+        assert torch.equal(s0, plain.su) and torch.equal(v0, plain.sv)
+        # The added 1e-10 is below a rounding.
+        torch.testing.assert_close(st, 2 * plain.su, rtol=4 * EPS32, atol=0.0)
+        torch.testing.assert_close(vt, 3 * plain.sv, rtol=4 * EPS32, atol=0.0)
