@@ -791,7 +791,6 @@ __device__ __forceinline__ void factor_tile(f32x4 m, float* d, float* s_inv, int
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       const float pivot = uniform_value(v[c], 4 * p + c);
-      if (bad == 0 && !(pivot > 0.0f)) bad = 4 * p + c + 1;
       rs[c] = inverse_sqrt(pivot);
       // The column times 1 / root (LAPACK's potf2 scaling); the diagonal,
       // which no other entry waits for, is the root with one correction (its
@@ -805,6 +804,17 @@ __device__ __forceinline__ void factor_tile(f32x4 m, float* d, float* s_inv, int
       const float root = pivot * rs[c];
       const float fixed = fmaf(fmaf(-root, root, pivot), 0.5f * rs[c], root);
       v[c] = r == 4 * p + c ? fixed : scaled;
+      // One scalar test for all that is not positive and finite, since this
+      // is the chain. An infinite pivot is its own root, which 0 = 1 / root
+      // does not give; its column is zero.
+      const uint32_t bits = __float_as_uint(pivot);
+      if (__builtin_expect(bits - 1u >= 0x7F7FFFFFu, 0)) {
+        if (bits == 0x7F800000u) {
+          if (r == 4 * p + c) v[c] = pivot;
+        } else if (bad == 0) {
+          bad = 4 * p + c + 1;
+        }
+      }
     }
     if (g == 0) {
       f32x4 q;

@@ -59,3 +59,40 @@ def test_fold(n):
     np.testing.assert_allclose(got, want, rtol=0, atol=bound)
     assert not np.triu(got, 1).any()
     np.testing.assert_array_equal(np.diagonal(got), 1.0)
+
+
+@pytest.mark.parametrize("j", [0, 3, 5, 17, 130, 300, 399])
+def test_infinite_pivot(j):
+    """An infinite diagonal entry is a pivot with an infinite root: its column
+    is zero below, and the rest is the factor of the matrix without it."""
+    import torch
+
+    from exl3_intel_arc_quantizer_amd.ldlq import cholesky_ex
+    n = 400
+    a = _spd(n, j)
+    a[j, j] = np.inf
+    L, info = cholesky_ex(torch.from_numpy(a).cuda())
+    L = L.cpu().numpy()
+    assert int(info.item()) == 0
+    assert L[j, j] == np.inf and not L[j + 1:, j].any()
+    keep = np.arange(n) != j
+    want = np.linalg.cholesky(a[np.ix_(keep, keep)].astype(np.float64))
+    np.testing.assert_allclose(L[np.ix_(keep, keep)], want, rtol=0,
+                               atol=1e-4 * np.abs(want).max())
+
+
+@pytest.mark.parametrize("n", [160, 520])
+def test_ill_conditioned(n):
+    """Eigenvalues over 2^18 (float32 still factors it): the backward error
+    stays that of n + 1 roundings an entry."""
+    import torch
+
+    from exl3_intel_arc_quantizer_amd.ldlq import cholesky_ex
+    rng = np.random.default_rng(n)
+    q, _ = np.linalg.qr(rng.standard_normal((n, n)))
+    a = ((q * 2.0 ** -rng.uniform(0.0, 18.0, n)) @ q.T)
+    a = (0.5 * (a + a.T)).astype(np.float32)
+    L, info = cholesky_ex(torch.from_numpy(a).cuda())
+    L = L.cpu().numpy().astype(np.float64)
+    assert int(info.item()) == 0
+    assert np.abs(L @ L.T - a).max() <= 4 * (n + 1) * 2.0 ** -24 * np.abs(a).max()
