@@ -348,6 +348,13 @@ struct GramPlan {
 // Measured, us, 192 / 128 at their best share count: 8192 x 4096 190 / 312,
 // 500 x 4096 24 / 36, 2048 x 2048 33 / 33, 8192 x 1024 37 / 39, 16384 x 512
 // 49 / 36.
+//
+// Partial tiles take no more memory than H itself, which a product and a sum
+// by a library would take as well, or 128 MiB. The bound costs wide inputs
+// alone, and those a few percent: 262,144 x 11,008 would share the tokens out
+// in four, 962 MiB beside an H of 462, for an estimated 34.0 ms against 34.7.
+constexpr int64_t GRAM_WORKSPACE = (int64_t)32 << 20;  // floats
+
 GramPlan gram_plan(int64_t tokens, int64_t d, int cus) {
   GramPlan best{};
   double least = 0.0;
@@ -359,6 +366,7 @@ GramPlan gram_plan(int64_t tokens, int64_t d, int cus) {
     for (int splits = 1; splits <= 32 && splits <= chunks; ++splits) {
       const int share = (chunks + splits - 1) / splits;
       if ((int64_t)share * (splits - 1) >= chunks) continue;  // an empty share
+      if (splits > 1 && splits * tiles * ts * ts > std::max(d * d, GRAM_WORKSPACE)) break;
       const double rounds = (double)((tiles * splits + cus - 1) / cus);
       double us = rounds * (share * cycles + 6000.0) / 2400.0;
       if (splits > 1) us += 5.0 + tiles * (double)ts * ts * 4.0 * 2.0 * splits / 4.0e6;

@@ -228,3 +228,16 @@ def test_ldlq_block_table_fields_match_the_header():
     body = text[text.index("typedef struct exl3_ldlq_block {"):text.index("} exl3_ldlq_block;")]
     fields = re.findall(r"int64_t (\w+);", body)
     assert tuple(fields) == _native.LDLQ_BLOCK_FIELDS
+
+
+def test_gram_workspace_is_bounded():
+    """Partial tiles of a Gram product take no more than the product itself,
+    or 128 MiB, whatever the token count."""
+    lib = _native.load_library()
+    for d in (8, 512, 1024, 3328, 4096, 5120, 8192, 11008, 12288, 14336):
+        for tokens in (1, 500, 8192, 16384, 65536, 262144, 1 << 24):
+            floats = lib.exl3_gram_workspace(tokens, d)
+            assert 0 <= floats <= max(d * d, 1 << 25), (tokens, d, floats)
+    assert lib.exl3_gram_workspace(16384, 512) > 0      # tokens are shared out
+    for tokens, d in ((0, 512), (8, 0), (8, 12), (8, 2 << 20)):
+        assert lib.exl3_gram_workspace(tokens, d) == -1
