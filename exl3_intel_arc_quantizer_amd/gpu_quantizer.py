@@ -622,7 +622,9 @@ class XPUTrellisEncoder:
         the records are built over the result arrays while the GPU encodes
         (1000 tiles of K=4: 2.11 ms, where building them afterwards took
         2.77); their values arrive at the end. ``search_seconds`` is then the
-        wall time until the encoder has finished."""
+        GPU's time for the batch (HIP events around it), beside which part of
+        ``postprocess_seconds`` runs: the parts may add up to more than the
+        total."""
         import torch
 
         arr = np.asarray(tiles, dtype=np.float32)
@@ -643,18 +645,19 @@ class XPUTrellisEncoder:
         t_transfer = time.perf_counter() - t0
 
         overlap = traceback_mode == "gpu_resident"
-        t_search0 = time.perf_counter()
         # The input has no NaN; the count only keeps encode_tensor from
         # reading one back in between.
         counter = (torch.zeros(1, dtype=torch.int32, device=raw_dev.device) if overlap else None)
+        stream = torch.cuda.current_stream(self.device_index)
+        started, encoded = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        if overlap:
+            started.record(stream)
         enc = self.encode_tensor(raw_dev, pre_permute=pre_permute, requested_b=requested_b,
                                  traceback_mode=traceback_mode, finalize=True,
                                  allocator_hook=allocator_hook, synchronize=not overlap,
                                  nan_count=counter)
-        encoded = None
         if overlap:
-            encoded = torch.cuda.Event()
-            encoded.record(torch.cuda.current_stream(self.device_index))
+            encoded.record(stream)
         tx = time.perf_counter()
         outs = [("idx", enc["indices"]), ("rec_perm", enc["reconstructed_perm"].to(torch.float16)),
                 ("rec", enc["reconstructed"]), ("path_cost", enc["path_cost"]),
@@ -685,9 +688,9 @@ class XPUTrellisEncoder:
                                                               list(rec_perm), list(packed))]
         post = time.perf_counter() - t_post0
 
-        if encoded is not None:
+        if overlap:
             encoded.synchronize()
-            enc["timings"]["search"] = time.perf_counter() - t_search0
+            enc["timings"]["search"] = started.elapsed_time(encoded) / 1e3
         tx = time.perf_counter()
         torch.cuda.synchronize(self.device_index)
         np.copyto(idx, host["idx"].numpy().view(np.uint16))

@@ -638,3 +638,24 @@ def test_large_batch_invariants(K):
     finally:
         enc.arena.release()
     _check_batch_invariants(x, bd, K, False, np.arange(0, 8192, 512))
+
+
+def test_search_seconds_is_the_encoders_time(monkeypatch):
+    """search_seconds counts the GPU's work and not the records that the host
+    builds beside it, however long they take."""
+    import time
+
+    from exl3_intel_arc_quantizer_amd import gpu_quantizer
+    plain = gpu_quantizer.EncodingResult
+
+    def slow(*args, **kwargs):
+        time.sleep(2e-3)
+        return plain(*args, **kwargs)
+
+    enc = gpu_quantizer.XPUTrellisEncoder(K=8)
+    tiles = np.random.default_rng(0).standard_normal((100, 256)).astype(np.float32)
+    enc.encode_batch_detailed(tiles)
+    monkeypatch.setattr(gpu_quantizer, "EncodingResult", slow)
+    bd = enc.encode_batch_detailed(tiles)
+    assert bd.postprocess_seconds >= 0.2
+    assert 0.0 < bd.search_seconds < 0.1 < bd.total_seconds
