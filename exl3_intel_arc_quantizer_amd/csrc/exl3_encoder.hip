@@ -1687,8 +1687,11 @@ static int resolve_policy(int policy) {
 // 182; K = 6, 1024 tiles 166 / 194, 1200 tiles 206 / 201; K = 7, 2048 tiles
 // 165 / 218, 3000 tiles 300 / 246; K = 8, 4096 tiles 190 / 283: the line is
 // 2 MiB of rows per step of the walk. At K = 1..3, whose rows are 16 KiB and
-// more and serve 3 to 8 steps, the per-row walk is as fast from 16 tiles on
-// (K = 3: 49 / 56 us at 16 tiles, 49 / 65 at 64).
+// more and serve 3 to 8 steps, the per-row walk is the faster one at every
+// size. Whole calls, us, streamed / per row at 1, 64 and 256 tiles: K = 1
+// 453 / 441, 509 / 471, 591 / 489; K = 2 431 / 426, 449 / 433, 518 / 459;
+// K = 3 417 / 409, 432 / 417, 482 / 457. There a policy alone reaches the
+// streamed kernel.
 static bool use_stream_traceback(const TbArgs& a, int policy) {
   if (policy == 1) return false;
   if (policy == 2) return true;

@@ -8,9 +8,11 @@
 //   damp_kernel         mean of the diagonal, damping and floor
 //
 // X^T X is symmetric: only tiles on and below the diagonal are computed and
-// each is stored twice, so a 4096-wide Hessian of 8192 tokens is 137 GFLOP
-// instead of the 275 of a general product, and the division by the token
-// count rides on the store instead of passes of its own.
+// each is stored twice, so a 4096-wide Hessian of 8192 tokens is 153 GFLOP
+// (253 whole tiles of 192; the triangle alone is 137) instead of the 275 of a
+// general product, and the division by the token count (a product with its
+// reciprocal, as torch divides by a host number) rides on the store instead
+// of passes of its own.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
@@ -58,7 +60,7 @@ __device__ __forceinline__ void lower_tile(int b, int& i, int& j) {
 // [c0, c1) of GR_K. v_mfma_f32_16x16x32 wants eight consecutive tokens of one
 // column in a lane, and X holds consecutive columns: a thread loads 8 tokens
 // x 8 columns (16-byte loads, coalesced along the columns; with 8-byte loads
-// an 8192 x 4096 Gram matrix took 220 us, 190 so), turns them with one v_perm
+// an 8192 x 4096 Gram matrix took 30 us more), turns them with one v_perm
 // per dword and stores eight 16-byte vectors (8 tokens of a column). Column
 // 8 q + j of an operand sits at vector j (TS / 8 + 2) + q of its token octet:
 // the stores of a wave are contiguous and the 16 lanes of a load phase hit 16
@@ -345,9 +347,9 @@ struct GramPlan {
 // workgroup each): rounds of workgroups times a share's chunks times a
 // chunk's cycles (measured at 1.0-1.4 us for 192 and 0.9 us for 128), plus
 // writing and reading the partial tiles where the tokens are shared out.
-// Measured, us, 192 / 128 at their best share count: 8192 x 4096 190 / 312,
-// 500 x 4096 24 / 36, 2048 x 2048 33 / 33, 8192 x 1024 37 / 39, 16384 x 512
-// 49 / 36.
+// Measured, us a call back to back, 192 / 128 at their best share count: 500 x
+// 4096 25 / 37, 8192 x 4096 164 / 297, 16384 x 5120 578 / 962, 2048 x 2048
+// 31 / 34, 8192 x 1024 36 / 32, 16384 x 512 47 / 40.
 //
 // Partial tiles take no more memory than H itself, which a product and a sum
 // by a library would take as well, or 128 MiB. The bound costs wide inputs

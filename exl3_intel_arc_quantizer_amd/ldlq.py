@@ -460,9 +460,12 @@ def _lanes_of(walks: List[_Traversal]) -> List[List[int]]:
     """Walks split into two lanes: those with the most blocks (the
     traversal's critical chain of calls) and the rest; one lane when every
     walk has the same length. On a 9B-class layer (down_proj 768 blocks,
-    the other six 256) this measured 1.22 s against 1.30 s for one lane,
-    and against 1.24-1.30 s for splits that move the smaller projections
-    into the first lane."""
+    the other six 256) this takes 1.02 s at K = 4 against 1.11 s for one
+    lane (K = 3 1.04 / 1.10, K = 6 1.07 / 1.15), and splits that move the
+    smaller projections into the first lane were 2-7 % slower. On a
+    2048-wide layer (352 and 128 blocks) the two are level: K = 3 292 / 293
+    ms, K = 4 292 / 297, K = 6 304 / 295. Two lanes vary more: about one
+    traversal in three took 12-25 % longer than these."""
     longest = max(len(w.blocks) for w in walks)
     lanes = [[i for i, w in enumerate(walks) if len(w.blocks) == longest],
              [i for i, w in enumerate(walks) if len(w.blocks) < longest]]
@@ -498,9 +501,12 @@ def _run_lockstep(walks: List[_Traversal], encode_tiles: TileEncoder,
     origin = torch.cuda.current_stream(device)
     encoders = [encode_tiles] + [encode_tiles.fork() for _ in groups[1:]]
     # Tracebacks by per-row tree loads: the streamed kernel reads whole rows,
-    # bandwidth the other lane's forward passes need (9B-class layer: 1.20 s
-    # against 1.23-1.26 s). Each adapter carries its own choice, so nothing
-    # process-wide changes and other threads' encodes are unaffected.
+    # bandwidth the other lane's forward passes need. Per row / by batch size
+    # (the streamed kernel where a call is small enough): 9B-class layer K = 4
+    # 1.020 / 1.031 s, K = 6 1.070 / 1.035; 2048-wide layer K = 4 292 / 286 ms,
+    # K = 5 305 / 296, K = 6 304 / 306; K <= 3 never streams. Each adapter
+    # carries its own choice, so nothing process-wide changes and other
+    # threads' encodes are unaffected.
     previous_policy = getattr(encode_tiles, "traceback_policy", None)
     for enc in encoders:
         enc.traceback_policy = "rows"

@@ -51,14 +51,13 @@ import torch
 
 from .hadamard import HAD_DIM, records
 
-# The kernels of exl3_output_scales / exl3_input_scales carry these values.
+# The values of the kernels of exl3_output_scales / exl3_input_scales.
 CODEBOOK_SCALE = 1.24371088     # the codebook's RMS, regularize.py:33
 OUT_SCALE_SKEW_CUTOFF = 0.15    # output scales only below this skew
 SKEW_FRACTION = 50              # the skew looks at the top 1/50 of the diagonal
 ZERO_FLOOR = 0.1                # scale used for an all-zero row or column
 EPS = 1e-10                     # added to every scale
 RMS_SLICE = 32                  # block_rms slice length
-_TINY = 1e-30                   # below this an RMS counts as zero
 
 
 def block_rms(x: torch.Tensor, dim: int, keepdim: bool = False,

@@ -26,10 +26,10 @@ extern "C" {
 int exl3_hadamard128(const float* in, float* out, int64_t rows, int64_t cols, int side,
                      void* stream);
 
-/* The two fused steps of regularize (regularize.py:171-181): each divides
- * the matrix by a scale vector and applies the blockwise Hadamard transform
- * in one pass over HBM, the arithmetic of a division (correctly rounded
- * fp32) followed by exl3_hadamard128.
+/* Division by a scale vector and the blockwise Hadamard transform in one pass
+ * over HBM, the arithmetic of a division (correctly rounded fp32) followed by
+ * exl3_hadamard128: the single steps that exl3_rotate and exl3_row_energy
+ * join (regularize.py:171-181), for a caller that wants them apart.
  * side = 1: out = (in / divisor[col]) @ H, divisor of `cols` floats (the
  *           fold of sv before H_r); slice_sumsq, if not NULL, receives the
  *           sum of squares of every 32-element slice of every output row,
