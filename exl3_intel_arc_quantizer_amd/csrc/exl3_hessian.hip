@@ -85,8 +85,7 @@ __device__ __forceinline__ void lower_tile(int b, int& i, int& j) {
 template <int TS, bool BF16, bool RUNS>
 __global__ void __launch_bounds__(GR_THREADS, 2)
     gram_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_t tokens, int64_t d,
-                float scale, float* __restrict__ h, float* __restrict__ parts, int tiles,
-                int chunks, int share, int run) {
+                float scale, float* h, float* parts, int tiles, int chunks, int share, int run) {
   constexpr int WI = TS / 32, WJ = TS / 64;          // 16 x 16 blocks of a wave
   constexpr int QP = TS / 8 + 2;                     // vectors of one column residue
   constexpr int OCT = 8 * QP;                        // vectors of one token octet
@@ -231,7 +230,8 @@ __global__ void __launch_bounds__(GR_THREADS, 2)
       float* total = parts ? parts + (int64_t)blockIdx.x * TS * TS : h + i0 * d + j0;
       int64_t ld = parts ? TS : d;
       // Not known to be the same in every run: the addresses of 4 WI WJ
-      // elements would otherwise stay in registers through the products.
+      // elements would otherwise stay in registers through the products. (So
+      // h and parts are not restrict: this is another pointer to them.)
       asm volatile("" : "+s"(total), "+s"(ld));
       float* own = total + row0 * ld + col0;
 #pragma unroll
